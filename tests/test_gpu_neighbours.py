@@ -1,0 +1,47 @@
+"""The neighbour search at the sizes where it can go wrong: one agent, agents
+in more than one block, more candidates in sight than an agent's list holds,
+exact ties in distance, one and sixteen neighbours, no and many segments."""
+import numpy as np
+import pytest
+
+from crowddynamics_amd import state as S
+from crowddynamics_amd.agents import empty_agents
+from crowddynamics_amd.device import DeviceAgents, Workspace, cell_capacity_for
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize('n,side,sight,k,n_seg', [
+    (1, 5.0, 3.0, 8, 2),      # no candidate at all
+    (17, 4.0, 3.0, 16, 0),    # one more agent than a block serves, all slots
+    (130, 2.5, 3.0, 1, 3),    # 129 candidates in sight, one over the list
+    (129, 1.9, 3.0, 16, 0),   # 128, exactly the list
+    (300, 3.0, 2.9, 8, 40),   # long lists and hidden neighbours
+    (400, 40.0, 3.0, 5, 17),  # sparse: most slots missing
+])
+def test_neighbours_equal_oracle(n, side, sight, k, n_seg):
+    rng = np.random.default_rng(n + k)
+    arr = empty_agents(n)
+    arr['position'] = rng.uniform(0, side, (n, 2))
+    arr['velocity'] = rng.normal(0, 1, (n, 2))
+    if n > 100:  # a lattice part: distances that tie exactly
+        m = n // 2
+        arr['position'][:m] = np.stack([np.arange(m) % 8, np.arange(m) // 8], 1) * 0.25
+    a = rng.uniform(0, side, (n_seg, 2))
+    segs = np.concatenate([a, a + rng.normal(0, 0.4, (n_seg, 2))], 1)
+    dev = DeviceAgents(arr)
+    ws = Workspace(n, cell_capacity_for(side, side, sight), 0, cell_slots=4)
+    got = S.find_nearest_neighbors(dev, sight, k, segs, ws)
+    want = O.nearest_neighbors(arr['position'], sight, k, segs)
+    assert np.array_equal(got.cpu().numpy(), want)
+    # the block list it leaves: the stable order by cell
+    pidx, cnt, off, shape, origin, cell_of = ws.block_list()
+    assert np.array_equal(pidx, np.argsort(cell_of, kind='stable'))
+    follower = rng.uniform(size=n) < 0.7
+    d, has = S.herding_interaction(dev, follower, got, 0.3, 0.4 * np.pi)
+    wd, wh = O.herding_interaction(follower, arr['position'], arr['velocity'], want, 0.3,
+                                   0.4 * np.pi)
+    assert np.array_equal(has.cpu().numpy(), wh)
+    # the sums keep their order: a few roundings of unit vectors
+    np.testing.assert_allclose(d.cpu().numpy(), wd, rtol=0, atol=1e-13)
