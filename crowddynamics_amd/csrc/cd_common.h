@@ -163,9 +163,10 @@ Layout make_layout(const cd_workspace_t *w) {
   // offsets it is built from
   L.order = take(4 * n);
   L.order_off = take(4 * cap);
-  // circular agents: the fused step's neighbour records, one per slot
-  // (NbrRec: 48 bytes in fp64, 32 in fp32)
-  L.rec = (w->model == CD_CIRCULAR) ? take(48 * slots) : -1;
+  // the fused step's neighbour records, one per slot (NbrRec: 48 bytes in
+  // fp64, 32 in fp32); three-circle agents, which the adjoint does not
+  // serve, keep them in its neighbour arrays (56 bytes per slot from e_pos)
+  L.rec = (w->model == CD_CIRCULAR) ? take(48 * slots) : L.e_pos;
   L.total = o;
   return L;
 }
@@ -237,7 +238,7 @@ struct Work {
   double2 *snap_ls, *snap_rs;
   double2 *snap_off;
   int *order, *order_off;  // force kernel's processing order (cell order when order_every > 0)
-  void *rec;               // circular agents: NbrRec of each slot, written by the fused step's K_a
+  void *rec;               // NbrRec of each slot, written by the fused step's K_a
   int cap, K, ntiles;
   int order_every;
 };
@@ -297,7 +298,7 @@ Work carve(const cd_workspace_t *w) {
   W.snap_rs = L.snap_rs >= 0 ? (double2 *)(b + L.snap_rs) : nullptr;
   W.snap_off = L.snap_off >= 0 ? (double2 *)(b + L.snap_off) : nullptr;
   W.order = (int *)(b + L.order);
-  W.rec = L.rec >= 0 ? (void *)(b + L.rec) : nullptr;
+  W.rec = (void *)(b + L.rec);
   W.order_off = (int *)(b + L.order_off);
   // only the agent-parallel force kernel follows the order
   W.order_every = (w->tile_x > 0 && w->tile_y > 0) ? 0 : (int)w->order_every;

@@ -473,7 +473,7 @@ constexpr int kTileThreads = 256;
 constexpr int kTileGroups = kTileThreads / 4;  // agents served at once
 constexpr int kTileMaxDim = 16;
 constexpr int kRegionMax = (kTileMaxDim + 2) * (kTileMaxDim + 2);
-constexpr int kWallTile = 256;
+constexpr int kWallTile = 128;  // wall segments staged in LDS at once (12 KB with frames and boxes)
 
 // LDS capacity (agents of a region): nine cells of up to 128 (circular) or
 // 56 (three-circle) agents fit, so a 3 x 3 region fits whenever no cell
@@ -578,11 +578,11 @@ struct Nbr {
   const double2 *off;   // ... or the snapshot's shoulder offsets (fused step)
 };
 
-// A slot's neighbour record (circular agents, fused step): the data a
-// candidate needs, written by the first kernel beside the slot's id, so the
-// force kernel reads it at one address with no id hop.  The same values as
-// the snapshot.  48 bytes in fp64, 32 in fp32 (the workspace holds 48 per
-// slot).
+// A slot's neighbour record (fused step): the data the gate of a candidate
+// needs, written by the first kernel beside the slot's id, so the force
+// kernel reads it at one address with no id hop.  The same values as the
+// snapshot; r is the radius of circular agents, tc_reach of three-circle
+// ones.  48 bytes in fp64, 32 in fp32 (the workspace holds 48 per slot).
 template <typename T>
 struct __attribute__((aligned(16))) NbrRec {
   double2 pos;
@@ -719,28 +719,28 @@ __device__ __forceinline__ TCView tc_select(bool take_b, const TCView &a, const 
 }
 
 // Three-circle: the reference evaluates the pair as interaction(min, max).
-__device__ __forceinline__ void pair_add_tc(int i, int j, const TCView &me, const TCView &other,
-                                            const Owner<double> &o, PairSum &ps) {
-  double px, py, m;
+// Agent i's side; false when the pair is out of sight.
+__device__ __forceinline__ bool pair_tc(int i, int j, const TCView &me, const TCView &other,
+                                        const Owner<double> &o, double &px, double &py,
+                                        double &m) {
   const bool sb = !(i < j);
-  const bool hit = pair_three_circle(tc_select(sb, me, other), tc_select(sb, other, me), sb, o,
-                                     px, py, m);
-  if (hit) {
-    ps.x.add(px);
-    ps.y.add(py);
-    ps.m.add(m);
-  }
+  return pair_three_circle(tc_select(sb, me, other), tc_select(sb, other, me), sb, o, px, py, m);
 }
 
 // The same in the fp32 mode (float force terms, double torque).
-__device__ __forceinline__ void pair_add_tc(int i, int j, const TCView &me, const TCView &other,
-                                            const Owner<float> &o, PairSum &ps) {
-  float px, py;
-  double m;
+__device__ __forceinline__ bool pair_tc(int i, int j, const TCView &me, const TCView &other,
+                                        const Owner<float> &o, float &px, float &py, double &m) {
   const bool sb = !(i < j);
-  const bool hit = pair_three_circle_f32(tc_select(sb, me, other), tc_select(sb, other, me), sb,
-                                         o, px, py, m);
-  if (hit) {
+  return pair_three_circle_f32(tc_select(sb, me, other), tc_select(sb, other, me), sb, o, px, py,
+                               m);
+}
+
+template <typename T>
+__device__ __forceinline__ void pair_add_tc(int i, int j, const TCView &me, const TCView &other,
+                                            const Owner<T> &o, PairSum &ps) {
+  T px, py;
+  double m;
+  if (pair_tc(i, j, me, other, o, px, py, m)) {
     ps.add(px, py);
     ps.m.add(m);
   }
@@ -910,19 +910,20 @@ __global__ void __launch_bounds__(256) k_step_begin(Agents<T> A, Work W, Batch B
     ss->time_tot += dt;
   }
   const bool bin = binning && g.ok;
-  // steps that rebuild the force kernel's processing order keep the slot ranks
-  const bool ranks = W.order_every > 0 && step % (uint64_t)W.order_every == 0ull;
   V2<T> *snap_vel = (V2<T> *)W.snap_vel;
   // an agent's snapshot and slot atomic (bin_begin), then its slot list
   // entry and neighbour record (bin_end)
   auto bin_begin = [&](int i, double2 pos, V2<T> vel, int &c, int &k, double &ri) {
-    ri = (MODEL == 0 && bin) ? A.radius[i] : 0.0;  // for the neighbour record
     W.snap_pos[i] = pos;
     snap_vel[i] = vel;
     if (MODEL) {
-      W.snap_ls[i] = A.ls[i];
-      W.snap_rs[i] = A.rs[i];
+      const double2 ls = A.ls[i], rs = A.rs[i];
+      ri = bin ? tc_reach(pos, ls, rs, A.r_t[i], A.r_s[i]) : 0.0;  // for the neighbour record
+      W.snap_ls[i] = ls;
+      W.snap_rs[i] = rs;
       W.snap_off[i] = shoulder_offset(A.r_ts[i], A.phi[i]);
+    } else {
+      ri = bin ? A.radius[i] : 0.0;
     }
     c = -1;
     k = 0;
@@ -938,9 +939,9 @@ __global__ void __launch_bounds__(256) k_step_begin(Agents<T> A, Work W, Batch B
         c = d.c0 + lc;
         W.cell_of[i] = c;
         k = atomicAdd(&count[c], 1);
-        // the slot: for the processing order, and (circular agents) for the
-        // force kernel, which skips the agent's own record by it
-        if (ranks || MODEL == 0) W.rank[i] = k;
+        // the slot: for the processing order, and for the force kernel,
+        // which skips the agent's own record by it
+        W.rank[i] = k;
       }
     }
   };
@@ -948,13 +949,11 @@ __global__ void __launch_bounds__(256) k_step_begin(Agents<T> A, Work W, Batch B
     if (c < 0) return;
     if (k < W.K) {
       W.ell_ids[c * W.K + k] = i;
-      if constexpr (MODEL == 0) {
-        NbrRec<T> rr;
-        rr.pos = pos;
-        rr.vel = vel;
-        rr.r = ri;
-        ((NbrRec<T> *)W.rec)[(size_t)c * W.K + k] = rr;
-      }
+      NbrRec<T> rr;
+      rr.pos = pos;
+      rr.vel = vel;
+      rr.r = ri;
+      ((NbrRec<T> *)W.rec)[(size_t)c * W.K + k] = rr;
     } else if (k == W.K) {  // the cell's list is full: its members are found by scanning cell_of
       atomicOr((unsigned long long *)&W.st->status, (unsigned long long)CD_STATUS_SLOTS_FULL);
     }
@@ -1092,10 +1091,6 @@ struct MemRow {
   const int *count;  // the count buffer of this binning
   Nbr<T> N;
   int c0, nx, ny, lx, ly, a0, a1;
-  // circular agents of the fused step: the slots' neighbour records, and the
-  // agent's own slot in its cell (the stencil's centre cell); else null
-  const NbrRec<T> *rec;
-  int self_slot;
   template <class F>
   __device__ __forceinline__ void visit(int self, int j, F &fn) const {
     if (j == self) return;
@@ -1141,48 +1136,7 @@ struct MemRow {
 #pragma unroll
       for (int k = 0; k < 9; ++k)
         so[k] = n[k] ? (gr[k / 3] + k % 3) * W.K - pre[k] : 0;
-      if constexpr (MODEL == 0) {
-        if (rec) {
-          // neighbour records: one load per candidate and no id hop; the
-          // agent's own record (centre cell k = 4, its slot) is skipped by
-          // its candidate index
-          const int sidx = self_slot >= 0 ? pre[4] + self_slot : -1;
-          // batches of kRecBatch candidates whose loads are issued together:
-          // four fp32 records, two fp64 ones (a batch of four fp64 records
-          // holds 40 registers, which made the fp64 kernel spill)
-          constexpr int kRecBatch = sizeof(T) == 8 ? 2 : 4;
-          for (int b = b0; b < b1; b += kRecBatch) {
-            int s[kRecBatch];
-#pragma unroll
-            for (int u = 0; u < kRecBatch; ++u) {
-              const int idx = b + u;
-              s[u] = -1;
-              if (idx < b1 && idx != sidx) {
-                int o = so[0];
-#pragma unroll
-                for (int k = 1; k < 9; ++k)
-                  if (idx >= pre[k]) o = so[k];
-                s[u] = o + idx;
-              }
-            }
-            NbrRec<T> rr[kRecBatch];
-#pragma unroll
-            for (int u = 0; u < kRecBatch; ++u)
-              if (s[u] >= 0) rr[u] = rec[s[u]];
-#pragma unroll
-            for (int u = 0; u < kRecBatch; ++u)
-              if (s[u] >= 0) fn(-1, rr[u].pos, rr[u].vel, rr[u].r);
-            // The batch's loads have all been consumed; waiting for them
-            // here says so to the compiler, which otherwise holds each
-            // record load of the next batch until the previous one arrives
-            // (their registers might, for all it knows, still be filling).
-            // s_waitcnt vmcnt(0), expcnt and lgkmcnt left at their maxima.
-            __builtin_amdgcn_s_waitcnt(0x0F70);
-          }
-          return;
-        }
-      }
-      // batches as for the records: four candidates, two fp64 circular ones
+      // four candidates; two fp64 circular ones (four held 40 registers)
       constexpr int kIdBatch = (MODEL == 0 && sizeof(T) == 8) ? 2 : 4;
       for (int b = b0; b < b1; b += kIdBatch) {
         int j[kIdBatch];
@@ -1214,7 +1168,12 @@ struct MemRow {
 #pragma unroll
           for (int u = 0; u < kIdBatch; ++u)
             if (j[u] >= 0 && j[u] != self) fn(j[u], xj[u], vj[u], rj[u]);
-          __builtin_amdgcn_s_waitcnt(0x0F70);  // as for the records
+          // The batch's loads have all been consumed; waiting for them here
+          // says so to the compiler, which otherwise holds each load of the
+          // next batch until the previous one arrives (their registers
+          // might, for all it knows, still be filling).
+          // s_waitcnt vmcnt(0), expcnt and lgkmcnt left at their maxima.
+          __builtin_amdgcn_s_waitcnt(0x0F70);
         } else {
           // one copy of the three-circle pair code for the batch (the id
           // picked by selects, not by indexing): an unrolled batch held
@@ -1226,7 +1185,7 @@ struct MemRow {
             for (int w = 1; w < kIdBatch; ++w) ju = u == w ? j[w] : ju;
             if (ju >= 0) visit(self, ju, fn);
           }
-          __builtin_amdgcn_s_waitcnt(0x0F70);  // as for the records
+          __builtin_amdgcn_s_waitcnt(0x0F70);  // as above
         }
       }
       return;
@@ -1356,15 +1315,60 @@ __device__ __forceinline__ Self<T> self_of(const Agents<T> &A, int i, double2 po
   return s;
 }
 
-// Pair and wall forces of agent i, served by L lanes (L = 2 to 64; q =
-// lane in the group): lane q takes part q of the stencil's candidates
+// Wall contacts of an agent served by L lanes (fused step): lane q of the
+// group takes every L-th of the walls from q, add(force x, force y, torque)
+// for each contact.  Every lane of the block calls this (have = false for
+// idle groups), so the staging barriers are uniform; the first kWallTile
+// segments are already staged.
+template <typename T, class Add>
+__device__ __forceinline__ void agent_walls(const FusedArgs &fa, const ScnDesc &d, double4 *sseg,
+                                            int model, int q, int L, bool have, double2 pos,
+                                            V2<T> vel, const WallSelf<T> &self, Add &&add) {
+  if (fa.wall_cells) {
+    // binned walls: only the segments listed for the agent's wall cell
+    // (a superset of those within its reach; outside the grid, none)
+    if (have) {
+      const double qx = (pos.x - fa.wall_minx) / fa.wall_cell;
+      const double qy = (pos.y - fa.wall_miny) / fa.wall_cell;
+      if (qx >= 0.0 && qy >= 0.0 && qx < (double)fa.wall_nx && qy < (double)fa.wall_ny) {
+        const int c = (int)qx * fa.wall_ny + (int)qy;
+        const int k0 = fa.wall_cells[c], k1 = fa.wall_cells[c + 1];
+        const int *ids = fa.wall_cells + (fa.wall_nx * fa.wall_ny + 1);
+        for (int k = k0 + q; k < k1; k += L) {
+          const double4 sg = fa.segs[d.w0 + ids[k]];
+          const double4 bx = make_double4(fmin(sg.x, sg.z), fmin(sg.y, sg.w),
+                                          fmax(sg.x, sg.z), fmax(sg.y, sg.w));
+          walls_each(self, model, pos, vel, &sg, nullptr, 1, add, 0, 1, &bx);
+        }
+      }
+    }
+    return;
+  }
+  const int nw = d.w1 - d.w0;
+  const double4 *sfrm = sseg + kWallTile, *sbox = sseg + 2 * kWallTile;
+  if (have) walls_each(self, model, pos, vel, sseg, sfrm, min(kWallTile, nw), add, q, L, sbox);
+  for (int w0 = kWallTile; w0 < nw; w0 += kWallTile) {  // more segments than staged
+    const int cnt = min(kWallTile, nw - w0);
+    __syncthreads();
+    stage_segs(fa.segs + d.w0 + w0, cnt, sseg);
+    __syncthreads();
+    if (have) walls_each(self, model, pos, vel, sseg, sfrm, cnt, add, q, L, sbox);
+  }
+  if (nw > kWallTile) {  // restore the first tile for the next agents
+    __syncthreads();
+    stage_walls(fa, d, sseg, true);
+    __syncthreads();
+  }
+}
+
+// Pair and wall forces of agent i in the tiled kernel, served by L lanes
+// (q = lane in the group): lane q takes part q of the stencil's candidates
 // (when `pairs`) and every L-th wall from q (fused step with walls).  Pair
 // and wall terms are summed exactly, so results do not depend on L.  Every
 // lane of the block calls this (have = false for idle groups), so the wall
-// staging barriers and the shuffles are uniform; the first kWallTile
-// segments are already staged.  Every lane of the group returns force
-// (torque) = self.f (self.tq) + (pairs + walls): the pair and wall terms
-// are one exact sum, rounded once.
+// staging barriers and the shuffles are uniform.  Every lane of the group
+// returns force (torque) = self.f (self.tq) + (pairs + walls): the pair and
+// wall terms are one exact sum, rounded once.
 template <typename T, int MODEL, bool FUSED, class Rows>
 __device__ __forceinline__ void agent_forces(const FusedArgs &fa, const ScnDesc &d,
                                              double4 *sseg, int L, bool have, bool pairs, int i,
@@ -1384,48 +1388,11 @@ __device__ __forceinline__ void agent_forces(const FusedArgs &fa, const ScnDesc 
       });
     }
   }
-  const bool walls = FUSED && (fa.flags & CD_USE_OBSTACLE);
-  if (walls) {  // wall contacts join the same exact sums
-    auto add = [&](T cx, T cy, double mm) {
+  if (FUSED && (fa.flags & CD_USE_OBSTACLE)) {  // wall contacts join the same exact sums
+    agent_walls(fa, d, sseg, MODEL, q, L, have, pos, vel, self.w, [&](T cx, T cy, double mm) {
       ps.add(cx, cy);
       if (MODEL) ps.m.add(mm);
-    };
-    if (fa.wall_cells) {
-      // binned walls: only the segments listed for the agent's wall cell
-      // (a superset of those within its reach; outside the grid, none)
-      if (have) {
-        const double qx = (pos.x - fa.wall_minx) / fa.wall_cell;
-        const double qy = (pos.y - fa.wall_miny) / fa.wall_cell;
-        if (qx >= 0.0 && qy >= 0.0 && qx < (double)fa.wall_nx && qy < (double)fa.wall_ny) {
-          const int c = (int)qx * fa.wall_ny + (int)qy;
-          const int k0 = fa.wall_cells[c], k1 = fa.wall_cells[c + 1];
-          const int *ids = fa.wall_cells + (fa.wall_nx * fa.wall_ny + 1);
-          for (int k = k0 + q; k < k1; k += L) {
-            const double4 sg = fa.segs[d.w0 + ids[k]];
-            const double4 bx = make_double4(fmin(sg.x, sg.z), fmin(sg.y, sg.w),
-                                            fmax(sg.x, sg.z), fmax(sg.y, sg.w));
-            walls_each(self.w, MODEL, pos, vel, &sg, nullptr, 1, add, 0, 1, &bx);
-          }
-        }
-      }
-    } else {
-      const int nw = d.w1 - d.w0;
-      const double4 *sfrm = sseg + kWallTile, *sbox = sseg + 2 * kWallTile;
-      if (have)
-        walls_each(self.w, MODEL, pos, vel, sseg, sfrm, min(kWallTile, nw), add, q, L, sbox);
-      for (int w0 = kWallTile; w0 < nw; w0 += kWallTile) {  // more segments than staged
-        const int cnt = min(kWallTile, nw - w0);
-        __syncthreads();
-        stage_segs(fa.segs + d.w0 + w0, cnt, sseg);
-        __syncthreads();
-        if (have) walls_each(self.w, MODEL, pos, vel, sseg, sfrm, cnt, add, q, L, sbox);
-      }
-      if (nw > kWallTile) {  // restore the first tile for the next agents
-        __syncthreads();
-        stage_walls(fa, d, sseg, true);
-        __syncthreads();
-      }
-    }
+    });
   }
   if constexpr (sizeof(T) == 4) ps.fold();
   // exact sums over the L lanes (butterfly: every lane ends with the totals)
@@ -1439,6 +1406,279 @@ __device__ __forceinline__ void agent_forces(const FusedArgs &fa, const ScnDesc 
   f.x += (T)ps.x.value();
   f.y += (T)ps.y.value();
   if (MODEL) tq += ps.m.value();
+}
+
+// What a wave of the direct kernel keeps in LDS: the queue of candidates
+// that passed the gate (slot or agent, and which of the wave's agents they
+// belong to), the agents' side of their pairs, and the agents' exact sums.
+// A sum is a Fix128 in three limbs (weights 2^-64, 2^-32 and 1, each
+// 64-bit, the last signed), so a term joins it by plain integer atomics
+// with no carry between them; limbs hold 2^32 terms.
+constexpr int kWaveAgents = 32;  // agents of a wave at 2 lanes each
+
+template <typename T, int MODEL>
+struct WaveLds {
+  static constexpr int U = sizeof(T) == 8 ? 2 : 4;  // candidates gated per lane and round
+  static constexpr int kQueue = 64 * (U + 1);       // fewer than 64 stay between rounds
+  static constexpr int NC = MODEL ? 3 : 2;          // force x, y (and torque)
+  int slot[kQueue];
+  int own[kQueue];
+  unsigned long long lo[NC][kWaveAgents], mid[NC][kWaveAgents], hi[NC][kWaveAgents];
+  int bad[NC][kWaveAgents];
+  T neg_mk[kWaveAgents], tau_0[kWaveAgents], mu[kWaveAgents], kappa[kWaveAgents],
+      damping[kWaveAgents], rtau_0[kWaveAgents];
+  double2 pos[MODEL ? 1 : kWaveAgents];
+  V2<T> vel[MODEL ? 1 : kWaveAgents];
+  double r[MODEL ? 1 : kWaveAgents];
+  int id[MODEL ? kWaveAgents : 1];
+
+  __device__ __forceinline__ void clear(int g) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      lo[c][g] = mid[c][g] = hi[c][g] = 0ull;
+      bad[c][g] = 0;
+    }
+  }
+  // Adds a term to component c of agent g: the Fix128 image of the term.
+  template <typename X>
+  __device__ __forceinline__ void add(int c, int g, X v) {
+    Fix128 t;
+    t.add(v);
+    if (t.bad) bad[c][g] = 1;
+    auto put = [](unsigned long long *p, unsigned long long x) {
+      __hip_atomic_fetch_add(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    if (sizeof(X) == 8) put(&lo[c][g], t.lo & 0xffffffffull);
+    else if ((t.lo & 0xffffffffull) != 0ull) put(&lo[c][g], t.lo & 0xffffffffull);
+    put(&mid[c][g], t.lo >> 32);
+    put(&hi[c][g], (unsigned long long)t.hi);
+  }
+  __device__ __forceinline__ double value(int c, int g) const {
+    Fix128 t;
+    t.lo = (mid[c][g] << 32) + lo[c][g];
+    t.hi = (long long)(hi[c][g] + (mid[c][g] >> 32) + (t.lo < lo[c][g] ? 1ull : 0ull));
+    t.bad = bad[c][g] != 0;
+    return t.value();
+  }
+  __device__ __forceinline__ Owner<T> owner(int g) const {
+    Owner<T> o;
+    o.neg_mk = neg_mk[g];
+    o.tau_0 = tau_0[g];
+    o.mu = mu[g];
+    o.kappa = kappa[g];
+    o.damping = damping[g];
+    o.rtau_0 = rtau_0[g];
+    return o;
+  }
+};
+
+// Orders a wave's own LDS accesses for the compiler (the hardware keeps them
+// in order).
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Pair terms of a wave's agents (L lanes each), into the wave's sums.  Every
+// lane calls this (on = false for idle lanes and without a valid binning).
+//
+// The lanes of an agent walk its 3 x 3 stencil, consecutive candidates on
+// consecutive lanes, and test each one with the gate of the pair function
+// (pair_circular_gate, pair_three_circle_gate): it needs only products and
+// passes every pair that can add a term.  Those that pass join the wave's
+// queue, and whenever 64 wait there (and at the end) every lane evaluates
+// one of them, for whichever agent it belongs to.  The sums are exact, so
+// neither who evaluates a pair nor when changes a result.
+//
+// Bound by the instructions of the walk and the gate.  A pair in sight adds
+// a term only if the two are on a collision course or touch: 3 % of the
+// candidates at cells of sight + 2 r, a fifth at 0.6 m.  Evaluating pairs
+// where they were met, a wave ran the pair function (300 instructions in
+// fp64) for nearly every candidate of its busiest lane.
+template <typename T, int MODEL, bool FUSED>
+__device__ __forceinline__ void wave_pairs(const Agents<T> &A, const Work &W, const Nbr<T> &N,
+                                           const int *count, const NbrRec<T> *rec,
+                                           const ScnDesc &d, int nx, int ny, int L, bool on,
+                                           int i, int c, int self_slot, double2 pos, V2<T> vel,
+                                           double ri, WaveLds<T, MODEL> &S) {
+  constexpr int U = WaveLds<T, MODEL>::U;
+  const int lane = threadIdx.x & 63;
+  const int lg = __builtin_ctz(L);  // L is a power of two
+  const int q = lane & (L - 1), g = lane >> lg;
+  // The stencil: candidate k-th cell's list begins at slot so[k] + pre[k];
+  // a cell holding more agents than slots has no candidates here (its
+  // members are found by scanning cell_of below).
+  int pre[10], so[9];
+  bool over = false;
+  int sidx = -1;  // the agent's own place among the candidates
+  {
+    const int lc = c - d.c0, lx = ny > 0 ? lc / ny : 0, ly = lc - lx * ny;
+    int n[9];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      const int ox = lx + r - 1;
+      const bool okx = on && ox >= 0 && ox < nx;
+      const int gr = d.c0 + ox * ny + ly - 1;  // the row's cell dy = -1
+      n[3 * r] = (okx && ly - 1 >= 0) ? count[gr] : 0;
+      n[3 * r + 1] = okx ? count[gr + 1] : 0;
+      n[3 * r + 2] = (okx && ly + 1 < ny) ? count[gr + 2] : 0;
+      so[3 * r] = (int)((unsigned)gr * (unsigned)W.K);  // (used where the cell is in the grid)
+      so[3 * r + 1] = so[3 * r] + W.K;
+      so[3 * r + 2] = so[3 * r + 1] + W.K;
+    }
+    pre[0] = 0;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      const bool full = n[k] > W.K;
+      over = over || full;
+      pre[k + 1] = pre[k] + (full ? 0 : n[k]);
+      so[k] -= pre[k];
+    }
+    if (FUSED && on && n[4] <= W.K) sidx = pre[4] + self_slot;
+  }
+  const int tot = pre[9];
+  int idx = q;
+  int jx = over ? d.a0 + q : d.a1;
+  int cnt = 0;  // candidates in the queue (the same in every lane)
+  auto push = [&](bool pass, int e) {
+    const unsigned long long m = __ballot(pass);
+    if (pass) {
+      const int at = cnt + (int)__builtin_amdgcn_mbcnt_hi(
+                               (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+      S.slot[at] = e;
+      S.own[at] = g;
+    }
+    cnt += __popcll(m);
+  };
+  auto gate = [&](double2 xj, V2<T> vj, double rj) -> bool {
+    if constexpr (MODEL == 0)
+      return pair_circular_gate<T>((T)(pos.x - xj.x), (T)(pos.y - xj.y), vel.x - vj.x,
+                                   vel.y - vj.y, (T)(ri + rj));
+    else
+      return pair_three_circle_gate<T>((T)(pos.x - xj.x), (T)(pos.y - xj.y), vel.x - vj.x,
+                                       vel.y - vj.y, (T)(ri + rj));
+  };
+  auto reach_of = [&](int j, double2 xj) -> double {
+    if constexpr (MODEL == 0)
+      return A.radius[j];
+    else
+      return tc_reach(xj, N.ls[j], N.rs[j], A.r_t[j], A.r_s[j]);
+  };
+  for (;;) {
+    bool last = false;
+    if (__any(idx < tot)) {
+      int s[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int at = idx + u * L;
+        s[u] = -1;
+        if (at < tot && at != sidx) {
+          int o = so[0];
+#pragma unroll
+          for (int k = 1; k < 9; ++k)
+            if (at >= pre[k]) o = so[k];
+          s[u] = o + at;
+        }
+      }
+      idx += U * L;
+      if constexpr (FUSED) {
+        NbrRec<T> rr[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (s[u] >= 0) rr[u] = rec[s[u]];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          push(s[u] >= 0 && gate(rr[u].pos, rr[u].vel, rr[u].r), s[u]);
+        // the batch's loads have all been consumed; waiting for them here
+        // says so to the compiler, which otherwise holds each load of the
+        // next batch until the previous one arrives
+        // (s_waitcnt vmcnt(0), expcnt and lgkmcnt left at their maxima)
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+      } else {
+        int j[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          j[u] = s[u] >= 0 ? W.ell_ids[s[u]] : i;
+        }
+        double2 xj[U];
+        V2<T> vj[U];
+        double rj[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (s[u] >= 0) {
+            xj[u] = N.pos[j[u]];
+            vj[u] = N.vel[j[u]];
+            rj[u] = reach_of(j[u], xj[u]);
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          push(s[u] >= 0 && j[u] != i && gate(xj[u], vj[u], rj[u]), ~j[u]);
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // as above
+      }
+    } else if (__any(jx < d.a1)) {
+      // members of overfull stencil cells: the agents of the scenario whose
+      // cell is one of them
+      bool pass = false;
+      if (jx < d.a1 && jx != i) {
+        const int gc = W.cell_of[jx];
+        if (gc >= d.c0 && count[gc] > W.K) {
+          const int l = gc - d.c0, ox = l / ny, own = c - d.c0, lx = own / ny;
+          const int dx = ox - lx, dy = (l - ox * ny) - (own - lx * ny);
+          if (dx >= -1 && dx <= 1 && dy >= -1 && dy <= 1) {
+            const double2 xj = N.pos[jx];
+            pass = gate(xj, N.vel[jx], reach_of(jx, xj));
+          }
+        }
+      }
+      push(pass, ~jx);
+      jx += L;
+    } else {
+      last = true;
+    }
+    while (cnt >= 64 || (last && cnt > 0)) {
+      const int m = min(cnt, 64);
+      cnt -= m;
+      wave_fence();
+      if (lane < m) {
+        const int e = S.slot[cnt + lane], o = S.own[cnt + lane];
+        if constexpr (MODEL == 0) {
+          double2 xj;
+          V2<T> vj;
+          double rj;
+          if (FUSED && e >= 0) {
+            const NbrRec<T> rr = rec[e];
+            xj = rr.pos;
+            vj = rr.vel;
+            rj = rr.r;
+          } else {
+            xj = N.pos[~e];
+            vj = N.vel[~e];
+            rj = A.radius[~e];
+          }
+          const double2 xi = S.pos[o];
+          const V2<T> vi = S.vel[o];
+          T px, py;
+          if (pair_circular<T>((T)(xi.x - xj.x), (T)(xi.y - xj.y), vi.x - vj.x, vi.y - vj.y,
+                               (T)(S.r[o] + rj), S.owner(o), px, py)) {
+            S.add(0, o, px);
+            S.add(1, o, py);
+          }
+        } else {
+          const int j = e >= 0 ? W.ell_ids[e] : ~e, me = S.id[o];
+          T px, py;
+          double m2;
+          if (pair_tc(me, j, tc_nbr(A, N, me), tc_nbr(A, N, j), S.owner(o), px, py, m2)) {
+            S.add(0, o, px);
+            S.add(1, o, py);
+            S.add(2, o, m2);
+          }
+        }
+      }
+      wave_fence();
+    }
+    if (last) break;
+  }
 }
 
 // Inputs of the integrator the force kernels of the fused step load early.
@@ -1501,16 +1741,18 @@ template <typename T, int MODEL, bool FUSED, bool ONE>
 __global__ void __launch_bounds__(256, MODEL == 0 ? 3 : 1) k_forces_direct(Agents<T> A, Work W, Batch B,
                                                        FusedArgs fa, int L, int reset,
                                                        int ordered) {
-  __shared__ double4 sseg[3 * kWallTile];
+  __shared__ double4 sseg[FUSED ? 3 * kWallTile : 1];
+  __shared__ WaveLds<T, MODEL> s_wave[4];
   const int2 sk = block_e_t<ONE>(B);
   const ScnDesc d = desc_t<ONE>(B, sk.x);
   // the walls' staging first: its wave waits for the segments, and its
   // loads would otherwise queue behind the agent's
   stage_walls(fa, d, sseg, FUSED);
-  const int per = (int)blockDim.x >> __builtin_ctz(L);  // L is a power of two
+  const int lg = __builtin_ctz(L);  // L is a power of two
+  const int per = (int)blockDim.x >> lg;
   // the agent: the next in index order, or in the processing order (an
   // entry outside the scenario, which a valid order never holds, serves none)
-  const int local = sk.y * per + ((int)threadIdx.x >> __builtin_ctz(L));
+  const int local = sk.y * per + ((int)threadIdx.x >> lg);
   int i = d.a0 + local;
   if (ordered && i < d.a1) i = W.order[i];
   const bool have = i >= d.a0 && i < d.a1;
@@ -1521,7 +1763,6 @@ __global__ void __launch_bounds__(256, MODEL == 0 ? 3 : 1) k_forces_direct(Agent
   vel.y = T(0);
   int c = d.c0;
   int self_slot = -1;
-  TCView me;
   Self<T> self;
   Tail<T> tail;
   // The agent's loads come first: they need only its index, not the
@@ -1532,8 +1773,7 @@ __global__ void __launch_bounds__(256, MODEL == 0 ? 3 : 1) k_forces_direct(Agent
     pos = A.pos[i];
     vel = A.vel[i];
     c = W.cell_of[i];
-    if (MODEL == 0 && FUSED) self_slot = W.rank[i];
-    if constexpr (MODEL == 1) me = tc_agent(A, i);
+    if (FUSED) self_slot = W.rank[i];
     self = self_of<T, MODEL>(A, i, pos);
     if (FUSED && lead) tail = tail_of(A, i);
   }
@@ -1548,20 +1788,55 @@ __global__ void __launch_bounds__(256, MODEL == 0 ? 3 : 1) k_forces_direct(Agent
   const bool ok = pairs_on & (valid != 0) & ((p ? oob1 : oob0) == 0);
   if (!FUSED && !ok) return;
   const double dt = FUSED ? dt_s : 0.0;
-  if (!ok) {
-    c = d.c0;
-    self_slot = -1;
+  // the agent's side of its pairs, for whichever lane evaluates them
+  WaveLds<T, MODEL> &S = s_wave[threadIdx.x >> 6];
+  const int g = (int)(threadIdx.x & 63) >> lg;
+  double ri = 0.0;
+  if (have) {
+    if constexpr (MODEL == 0)
+      ri = self.w.r;
+    else
+      ri = tc_reach(pos, self.w.ls, self.w.rs, self.w.rt, self.w.rsr);
   }
-  const int lc = c - d.c0, lx = ny > 0 ? lc / ny : 0, ly = lc - lx * ny;
-  const MemRow<T, MODEL> rows{A, W, W.count + (size_t)p * W.cap,
-                              FUSED ? nbr_snapshot<T>(W) : nbr_agents(A),
-                              d.c0, nx, ny, lx, ly, d.a0, d.a1,
-                              (MODEL == 0 && FUSED) ? (const NbrRec<T> *)W.rec : nullptr,
-                              self_slot};
-  __syncthreads();  // walls staged
-  V2<T> f;
-  double tq;
-  agent_forces<T, MODEL, FUSED>(fa, d, sseg, L, have, ok, i, pos, vel, me, self, rows, f, tq);
+  if ((threadIdx.x & (L - 1)) == 0) S.clear(g);
+  if (lead) {
+    S.neg_mk[g] = self.o.neg_mk;
+    S.tau_0[g] = self.o.tau_0;
+    S.mu[g] = self.o.mu;
+    S.kappa[g] = self.o.kappa;
+    S.damping[g] = self.o.damping;
+    S.rtau_0[g] = self.o.rtau_0;
+    if constexpr (MODEL == 0) {
+      S.pos[g] = pos;
+      S.vel[g] = vel;
+      S.r[g] = ri;
+    } else {
+      S.id[g] = i;
+    }
+  }
+  wave_fence();
+  if (ok)
+    wave_pairs<T, MODEL, FUSED>(A, W, FUSED ? nbr_snapshot<T>(W) : nbr_agents(A),
+                                W.count + (size_t)p * W.cap, (const NbrRec<T> *)W.rec, d, nx, ny,
+                                L, have, i, c, self_slot, pos, vel, ri, S);
+  if (FUSED && (fa.flags & CD_USE_OBSTACLE)) {  // wall contacts join the same exact sums
+    __syncthreads();  // walls staged
+    agent_walls(fa, d, sseg, MODEL, (int)threadIdx.x & (L - 1), L, have, pos, vel, self.w,
+                [&](T cx, T cy, double mm) {
+                  S.add(0, g, cx);
+                  S.add(1, g, cy);
+                  if constexpr (MODEL == 1) S.add(2, g, mm);
+                });
+  }
+  wave_fence();
+  // force (torque) += pairs + walls: one exact sum, rounded once
+  V2<T> f = self.f;
+  double tq = self.tq;
+  if (lead) {
+    f.x += (T)S.value(0, g);
+    f.y += (T)S.value(1, g);
+    if constexpr (MODEL == 1) tq += S.value(2, g);
+  }
   Red r;
   r.init();
   agent_finish<T, MODEL, FUSED>(A, fa, i, lead, f, tq, pos, vel, tail, dt, reset, r);
@@ -1714,7 +1989,7 @@ __device__ void cell_from_memory(const Agents<T> &A, const Work &W, const FusedA
                                  int ly, const TileCtx<T> &cx, Red &red, bool pairs = true,
                                  int part = 0, int nb = 1) {
   const int gc = d.c0 + lx * ny + ly;
-  const MemRow<T, MODEL> rows{A, W, cx.count, cx.N, d.c0, nx, ny, lx, ly, d.a0, d.a1, nullptr, -1};
+  const MemRow<T, MODEL> rows{A, W, cx.count, cx.N, d.c0, nx, ny, lx, ly, d.a0, d.a1};
   for (int j0 = d.a0 + part * kTileGroups; j0 < d.a1; j0 += nb * kTileGroups) {
     const int i = j0 + (threadIdx.x >> 2);
     const bool have = i < d.a1 && (!pairs || W.cell_of[i] == gc);
