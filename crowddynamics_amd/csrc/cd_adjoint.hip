@@ -684,7 +684,7 @@ int diff_prepare(const Agents<double> &A, const cd_step_params_t *p, const Work 
     if ((rc = launch_reduce(A, W, B, L.blocks_f, true, s))) return rc;
   if (adaptive) hipLaunchKernelGGL(k_adj_dt, dim3(1), dim3(kBS), 0, s, W, B, 1);
   if (pairs) {
-    hipLaunchKernelGGL(k_bin_insert, dim3(L.blocks_f), dim3(kBS), 0, s, (const double2 *)A.pos,
+    hipLaunchKernelGGL((k_bin_insert<double, false>), dim3(L.blocks_f), dim3(kBS), 0, s, A, 0,
                        p->cell_size, W, B, 1);
     hipLaunchKernelGGL(k_cell_gather<double>, dim3(grid_for((int64_t)W.cap * 64, kBS)),
                        dim3(kBS), 0, s, A, W);

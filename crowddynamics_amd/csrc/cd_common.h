@@ -163,8 +163,8 @@ Layout make_layout(const cd_workspace_t *w) {
   // offsets it is built from
   L.order = take(4 * n);
   L.order_off = take(4 * cap);
-  // the fused step's neighbour records, one per slot (NbrRec: 48 bytes in
-  // fp64, 32 in fp32); three-circle agents, which the adjoint does not
+  // the force kernels' neighbour records, one per slot (NbrRec: 48 bytes in
+  // fp64, 40 in fp32); three-circle agents, which the adjoint does not
   // serve, keep them in its neighbour arrays (56 bytes per slot from e_pos)
   L.rec = (w->model == CD_CIRCULAR) ? take(48 * slots) : L.e_pos;
   L.total = o;
@@ -238,7 +238,7 @@ struct Work {
   double2 *snap_ls, *snap_rs;
   double2 *snap_off;
   int *order, *order_off;  // force kernel's processing order (cell order when order_every > 0)
-  void *rec;               // NbrRec of each slot, written by the fused step's K_a
+  void *rec;               // NbrRec of each slot, written by K_a
   int cap, K, ntiles;
   int order_every;
 };
@@ -501,22 +501,25 @@ __device__ Red reduce_partials(const Work &W, const ScnDesc &d) {
   return block_reduce(r);
 }
 
+// A slot keeps each field in an image that merges by max (the minima
+// complemented), so lanes holding different fields run one instruction.
+__device__ __forceinline__ unsigned long long red_up(int field, unsigned long long v) {
+  return field <= R_MINY ? ~v : v;
+}
+
 // Merges a block's reduction into a scenario's slot: exact and independent
 // of order (min / max of ordered bits, or of the non-negative speed bits).
 __device__ __forceinline__ void acc_merge(unsigned long long *acc, const Red &r) {
-  atomicMin(&acc[R_MINX], r.v[R_MINX]);
-  atomicMin(&acc[R_MINY], r.v[R_MINY]);
-  atomicMax(&acc[R_MAXX], r.v[R_MAXX]);
-  atomicMax(&acc[R_MAXY], r.v[R_MAXY]);
-  atomicMax(&acc[R_VMAX], r.v[R_VMAX]);
-  atomicMax(&acc[R_V0MAX], r.v[R_V0MAX]);
-  atomicMax(&acc[R_NONFINITE], r.v[R_NONFINITE]);
+#pragma unroll
+  for (int k = 0; k < R_COUNT; ++k) atomicMax(&acc[k], red_up(k, r.v[k]));
 }
 
 __device__ __forceinline__ void acc_reset(unsigned long long *acc) {
   Red r;
   r.init();
-  for (int k = 0; k < R_COUNT; ++k) acc[k] = r.v[k];
+#pragma unroll
+  for (int k = 0; k < R_COUNT; ++k) acc[k] = red_up(k, r.v[k]);
+  acc[R_COUNT] = 0ull;
 }
 
 // Sub-slot `sub` of reduction slot `slot` of scenario `scn`.
@@ -524,26 +527,49 @@ __device__ __forceinline__ unsigned long long *acc_at(const Work &W, int scn, in
   return W.acc + ((size_t)(scn * 2 + slot) * kAccSub + sub) * 8;
 }
 
-// Wave-wide reduction; every lane returns the wave's result.  `first`: the
-// lanes hold the identity except every first-th one (a power of two), so
-// the exchanges below that distance are skipped.
-__device__ __forceinline__ Red wave_reduce(Red r, int first = 1) {
-  for (int o = 32; o >= first; o >>= 1) {
-    unsigned long long u[R_COUNT];
+// The maximum over the lanes of equal index mod 8 (every lane gets its own).
+__device__ __forceinline__ unsigned long long max_by_field(unsigned long long v) {
 #pragma unroll
-    for (int k = 0; k < R_COUNT; ++k) u[k] = shfl_xor64(r.v[k], o);
-    r.combine(u);
+  for (int o = 8; o < 64; o <<= 1) v = max(v, shfl_xor64(v, o));
+  return v;
+}
+
+// The reduction held by a scenario's slot, combined by each wave on its own
+// (no block barrier); every thread returns it.  Lane l takes field l mod 8
+// of every eighth sub-slot, so the lanes combine one value in three
+// exchanges.  (A lane that took whole sub-slots had seven values to combine
+// in six exchanges each: 250 instructions.)
+__device__ __forceinline__ Red acc_read(const Work &W, int scn, int slot) {
+  static_assert(kAccSub % 8 == 0 && R_COUNT < 8, "a lane per field");
+  const unsigned long long *acc = acc_at(W, scn, slot, 0) + (threadIdx.x & 63);
+  unsigned long long v = 0ull;
+#pragma unroll
+  for (int k = 0; k < kAccSub / 8; ++k) v = max(v, acc[64 * k]);
+  v = max_by_field(v);
+  Red r;
+#pragma unroll
+  for (int k = 0; k < R_COUNT; ++k) {
+    const unsigned lo = __builtin_amdgcn_readlane((unsigned)v, k);
+    const unsigned hi = __builtin_amdgcn_readlane((unsigned)(v >> 32), k);
+    r.v[k] = red_up(k, ((unsigned long long)hi << 32) | lo);
   }
   return r;
 }
 
-// The reduction held by a scenario's slot, combined by each wave on its own
-// (no block barrier); every thread returns it.
-__device__ __forceinline__ Red acc_read(const Work &W, int scn, int slot) {
-  Red r;
-  r.init();
-  for (int sub = threadIdx.x & 63; sub < kAccSub; sub += 64) r.combine(acc_at(W, scn, slot, sub));
-  return wave_reduce(r);
+// A wave's agents join a sub-slot of a scenario's slot: agent g's reduction
+// is put into `buf` (8 words each) by the lane that holds it, then lane l
+// takes field l mod 8 of every eighth agent and one atomic merges all fields.
+__device__ __forceinline__ void red_put(unsigned long long *buf, int g, const Red &r) {
+#pragma unroll
+  for (int k = 0; k < R_COUNT; ++k) buf[8 * g + k] = red_up(k, r.v[k]);
+}
+__device__ __forceinline__ void red_merge(unsigned long long *acc, const unsigned long long *buf,
+                                          int agents) {
+  const int lane = threadIdx.x & 63, field = lane & 7;
+  unsigned long long v = 0ull;  // the least image
+  for (int g = lane >> 3; g < agents; g += 8) v = max(v, buf[8 * g + field]);
+  v = max_by_field(v);
+  if (lane < R_COUNT) atomicMax(&acc[lane], v);
 }
 
 __device__ __forceinline__ double red_vmax(const unsigned long long *v) {
@@ -668,21 +694,57 @@ __device__ __forceinline__ int cell_of_pos(double2 p, const Grid &g, double cell
 // K_a / K_b: per-cell slot lists
 // ---------------------------------------------------------------------------
 
+// A slot's neighbour record: what the force kernels need of a candidate,
+// written beside the slot's id by the kernel that bins it, so a candidate
+// costs one load with no id hop.  gate: gate_reach of the agent's body; r:
+// the radius of circular agents (their pair function needs no more).  48
+// bytes in fp64, 40 in fp32 (the workspace holds 48 per slot).
+template <typename T>
+struct __attribute__((aligned(sizeof(T) == 8 ? 16 : 8))) NbrRec {
+  double x, y;
+  V2<T> vel;
+  double r;
+  int id;
+  float gate;
+};
+static_assert(sizeof(NbrRec<double>) == 48 && sizeof(NbrRec<float>) == 40, "NbrRec layout");
+
+template <typename T>
+__device__ __forceinline__ NbrRec<T> nbr_rec(int i, double2 pos, V2<T> vel, double reach) {
+  NbrRec<T> n;
+  n.x = pos.x;
+  n.y = pos.y;
+  n.vel = vel;
+  n.r = reach;
+  n.id = i;
+  n.gate = gate_reach(reach);
+  return n;
+}
+
+// How far agent i's body reaches from its centre.
+template <typename T>
+__device__ __forceinline__ double body_reach(const Agents<T> &A, int model, int i, double2 pos) {
+  return model ? tc_reach(pos, A.ls[i], A.rs[i], A.r_t[i], A.r_s[i]) : A.radius[i];
+}
+
 // Binning of a scenario's agents with the grid of its reduced partials:
 // publishes the grid (one thread per scenario) and, when `binning`, inserts
 // the agents into their cells' slot lists (slots beyond cell_slots are not
 // stored; the cell count tells).  Cell indices are global: scenario base +
 // local cell.  p0: the position of the block's first agent, loaded early.
-__device__ __forceinline__ void bin_scenario(const double2 *pos, double2 p0, double cell,
-                                             const Work &W, const ScnDesc &d, ScnState *ss,
-                                             int2 sk, const Red &r, int binning) {
+// REC: the slots' neighbour records too.
+template <typename T, bool REC>
+__device__ __forceinline__ void bin_scenario(const Agents<T> &A, int model, double2 p0,
+                                             double cell, const Work &W, const ScnDesc &d,
+                                             ScnState *ss, int2 sk, const Red &r, int binning) {
   const int stride = d.nf * blockDim.x;
   const int i0 = d.a0 + sk.y * blockDim.x + threadIdx.x;
   const Grid g = grid_of(r, cell, d.ccap);
   if (sk.y == 0 && threadIdx.x == 0) publish_grid(W, ss, r, g, binning != 0, d.a1 > d.a0, 0);
   if (!binning || !g.ok) return;
   for (int i = i0; i < d.a1; i += stride) {
-    const int lc = cell_of_pos(i == i0 ? p0 : pos[i], g, cell);
+    const double2 p = i == i0 ? p0 : A.pos[i];
+    const int lc = cell_of_pos(p, g, cell);
     if (lc < 0) {  // positions changed after the bounding box was reduced
       atomicOr(&ss->oob[0], 1);
       W.cell_of[i] = -1;
@@ -691,24 +753,29 @@ __device__ __forceinline__ void bin_scenario(const double2 *pos, double2 p0, dou
     const int c = d.c0 + lc;
     W.cell_of[i] = c;
     const int k = atomicAdd(&W.count[c], 1);
-    if (k < W.K)
+    if (k < W.K) {
       W.ell_ids[c * W.K + k] = i;
-    else if (k == W.K)  // the cell's list is full: its members are found by scanning cell_of
+      if constexpr (REC)
+        ((NbrRec<T> *)W.rec)[(size_t)c * W.K + k] =
+            nbr_rec<T>(i, p, A.vel[i], body_reach(A, model, i, p));
+    } else if (k == W.K) {  // the cell's list is full: its members are found by scanning cell_of
       atomicOr((unsigned long long *)&W.st->status, (unsigned long long)CD_STATUS_SLOTS_FULL);
+    }
   }
 }
 
 // K_a of the operator paths: combine the scenario's partials, then
 // bin_scenario.
-__global__ void __launch_bounds__(256) k_bin_insert(const double2 *pos, double cell, Work W,
+template <typename T, bool REC>
+__global__ void __launch_bounds__(256) k_bin_insert(Agents<T> A, int model, double cell, Work W,
                                                     Batch B, int binning) {
   const int2 sk = block_f(B);
   const ScnDesc d = desc_of(B, sk.x);
   ScnState *ss = &B.sst[sk.x];
   const int i0 = d.a0 + sk.y * blockDim.x + threadIdx.x;
-  const double2 p0 = (binning && i0 < d.a1) ? pos[i0] : make_double2(0.0, 0.0);
+  const double2 p0 = (binning && i0 < d.a1) ? A.pos[i0] : make_double2(0.0, 0.0);
   const Red r = reduce_partials(W, d);
-  bin_scenario(pos, p0, cell, W, d, ss, sk, r, binning);
+  bin_scenario<T, REC>(A, model, p0, cell, W, d, ss, sk, r, binning);
 }
 
 // K_b: one wave per cell of the workspace grid.  Orders the cell's slot list

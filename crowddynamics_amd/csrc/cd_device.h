@@ -331,30 +331,34 @@ struct Owner {
 // hypot) feeds the contact force.  Only the pairs within 2^-40 of a
 // threshold take the library hypot.
 
-// Whether the pair below can add a term: false only where pair_circular
-// returns false or zeros.  The products are its own, so their signs are
-// those it branches on: a social term needs a discriminant above zero and a
-// time to collision above zero, (b - ds) / a with ds >= 0, hence b > 0.  In
-// contact or near it (fp64: as `clear` below; fp32: within 2^-16 of r_tot,
-// above the error of its distance) the pair passes; so does any pair whose
-// velocities give NaN there.  The sight limit takes the same margins.
-template <typename T>
-__device__ __forceinline__ bool pair_circular_gate(T x, T y, T vx, T vy, T r_tot) {
-  if constexpr (std::is_same<T, double>::value) {
-    const double s = x * x + y * y, rs = kSightSoc + r_tot, r2 = r_tot * r_tot;
-    const double a = vx * vx + vy * vy;
-    const double b = -(x * vx + y * vy);
-    const double disc = b * b - a * (s - r2);
-    return s <= (rs * rs) * (1.0 + kGate) && ((disc > 0.0 && b > 0.0) || s <= r2 * (1.0 + kGate));
-  } else {
-    const float d2 = __builtin_fmaf(x, x, y * y), rs = float(kSightSoc) + r_tot;
-    const float a = __builtin_fmaf(vx, vx, vy * vy);
-    const float b = -__builtin_fmaf(x, vx, y * vy);
-    const float c = __builtin_fmaf(-r_tot, r_tot, d2);
-    const float disc = __builtin_fmaf(b, b, -(a * c));
-    return d2 <= (rs * rs) * (1.0f + 0x1p-16f) &&
-           ((disc > 0.0f && b > 0.0f) || d2 <= (r_tot * r_tot) * (1.0f + 0x1p-16f));
-  }
+// The gate of a pair: false only where the pair function (pair_circular,
+// pair_three_circle and their fp32 forms) returns false or zeros.  (x, y)
+// and (vx, vy) are the centres' and velocities' differences in float, R the
+// sum of the agents' gate_reach.  Each agent lies in a disc about its centre;
+// a pair adds a term only if the discs touch, c = |x|^2 - R^2 < 0, or will,
+// b = -x v > 0 and b^2 - a c > 0 (in the pair function: tau = (b - ds) / a >
+// 0), and if they are within sight of each other, |x| < 3 + R.
+//
+// gate_reach grows a body's reach by m = 2^-7 m, so every test holds for what
+// the pair function computes: where the gate finds the discs passing or
+// parting, the bodies' own distance of closest approach exceeds their radii's
+// sum by 2 m.  A discriminant is then below -a (2 R m + m^2), while its
+// rounding errors, here and there, are below 2^-18 a |x|^2 in float
+// (three-circle: |x| at most doubles from centres to parts), and |x| < 3 + R.
+// A relative speed whose square underflows in float collides after 10^18 s.
+//
+// min and max take the other operand for NaN: with NaN in the velocities a
+// pair passes if it touches (and NaN joins the sum there).
+__device__ __forceinline__ bool pair_gate(float x, float y, float vx, float vy, float R) {
+  const float nb = __builtin_fmaf(x, vx, y * vy);
+  const float a = __builtin_fmaf(vx, vx, vy * vy);
+  const float c = __builtin_fmaf(-R, R, __builtin_fmaf(x, x, y * y));
+  const float disc = __builtin_fmaf(nb, nb, -(a * c));
+  const float sight = __builtin_fmaf(2.0f * float(kSightSoc), R, float(kSightSoc * kSightSoc)) - c;
+  return __builtin_fminf(sight, __builtin_fmaxf(__builtin_fminf(disc, -nb), -c)) > 0.0f;
+}
+__device__ __forceinline__ float gate_reach(double reach) {
+  return (float)(fabs(reach) * (1.0 + 0x1p-16) + 0x1p-7);
 }
 
 template <typename T>
@@ -536,32 +540,6 @@ __device__ __forceinline__ double tc_reach(double2 p, double2 ls, double2 rs, do
   const double lx = ls.x - p.x, ly = ls.y - p.y, rx = rs.x - p.x, ry = rs.y - p.y;
   const double o2 = fmax(lx * lx + ly * ly, rx * rx + ry * ry);
   return fmax(fabs(r_t), __builtin_amdgcn_sqrt(o2) * (1.0 + 0x1p-20) + fabs(r_s));
-}
-
-// Whether a three-circle pair can add a term: false only where
-// pair_three_circle (pair_three_circle_f32) returns false or zeros.  (x, y)
-// and (vx, vy) are the torsos' differences and R the sum of their tc_reach,
-// so the agents lie in two discs whose centres are sqrt(s) apart.
-//  * Discs apart (s > R^2): no contact.
-//  * Then moving apart (b <= 0): no part pair collides later; what its
-//    discriminant or its time to collision is, one of them is not positive.
-//  * The line of motion passing the centre by more than R (m0 > R, m0^2 a =
-//    s a - b^2): no part pair collides, its discriminant is negative.
-// The margin e makes each test hold for the computed values: parts then
-// stay apart by at least e / 2 sqrt(s), so a part pair's exact discriminant
-// is below -a s e^2 / 4, and its rounding error is below 2^-46 a s in fp64
-// (fp32: 2^-18 a s; s at most quadruples from torsos to parts).  Comparisons
-// with NaN pass.
-template <typename T>
-__device__ __forceinline__ bool pair_three_circle_gate(T x, T y, T vx, T vy, T R) {
-  constexpr T e = sizeof(T) == 8 ? T(0x1p-20) : T(0x1p-6);
-  const T s = x * x + y * y, r2 = R * R, rs = T(kSightSoc) + R;
-  const T a = vx * vx + vy * vy;
-  const T b = -(x * vx + y * vy);
-  const bool apart = s > r2 * (T(1) + e);
-  const bool past = b * b - a * (s - r2) < -e * (a * s);
-  const bool far = s > (rs * rs) * (T(1) + e);
-  return !(far || (apart && (b <= T(0) || past)));
 }
 
 // interaction_agent_agent_three_circle (core/interactions.py:73-104) in the

@@ -578,19 +578,6 @@ struct Nbr {
   const double2 *off;   // ... or the snapshot's shoulder offsets (fused step)
 };
 
-// A slot's neighbour record (fused step): the data the gate of a candidate
-// needs, written by the first kernel beside the slot's id, so the force
-// kernel reads it at one address with no id hop.  The same values as the
-// snapshot; r is the radius of circular agents, tc_reach of three-circle
-// ones.  48 bytes in fp64, 32 in fp32 (the workspace holds 48 per slot).
-template <typename T>
-struct __attribute__((aligned(16))) NbrRec {
-  double2 pos;
-  V2<T> vel;
-  double r;
-};
-static_assert(sizeof(NbrRec<double>) == 48 && sizeof(NbrRec<float>) == 32, "NbrRec layout");
-
 template <typename T>
 __host__ __device__ __forceinline__ Nbr<T> nbr_agents(const Agents<T> &A) {
   Nbr<T> N;
@@ -910,6 +897,8 @@ __global__ void __launch_bounds__(256) k_step_begin(Agents<T> A, Work W, Batch B
     ss->time_tot += dt;
   }
   const bool bin = binning && g.ok;
+  // steps that rebuild the force kernel's processing order keep the slot ranks
+  const bool ranks = W.order_every > 0 && step % (uint64_t)W.order_every == 0ull;
   V2<T> *snap_vel = (V2<T> *)W.snap_vel;
   // an agent's snapshot and slot atomic (bin_begin), then its slot list
   // entry and neighbour record (bin_end)
@@ -918,7 +907,7 @@ __global__ void __launch_bounds__(256) k_step_begin(Agents<T> A, Work W, Batch B
     snap_vel[i] = vel;
     if (MODEL) {
       const double2 ls = A.ls[i], rs = A.rs[i];
-      ri = bin ? tc_reach(pos, ls, rs, A.r_t[i], A.r_s[i]) : 0.0;  // for the neighbour record
+      ri = bin ? tc_reach(pos, ls, rs, A.r_t[i], A.r_s[i]) : 0.0;
       W.snap_ls[i] = ls;
       W.snap_rs[i] = rs;
       W.snap_off[i] = shoulder_offset(A.r_ts[i], A.phi[i]);
@@ -939,9 +928,7 @@ __global__ void __launch_bounds__(256) k_step_begin(Agents<T> A, Work W, Batch B
         c = d.c0 + lc;
         W.cell_of[i] = c;
         k = atomicAdd(&count[c], 1);
-        // the slot: for the processing order, and for the force kernel,
-        // which skips the agent's own record by it
-        W.rank[i] = k;
+        if (ranks) W.rank[i] = k;
       }
     }
   };
@@ -949,11 +936,7 @@ __global__ void __launch_bounds__(256) k_step_begin(Agents<T> A, Work W, Batch B
     if (c < 0) return;
     if (k < W.K) {
       W.ell_ids[c * W.K + k] = i;
-      NbrRec<T> rr;
-      rr.pos = pos;
-      rr.vel = vel;
-      rr.r = ri;
-      ((NbrRec<T> *)W.rec)[(size_t)c * W.K + k] = rr;
+      ((NbrRec<T> *)W.rec)[(size_t)c * W.K + k] = nbr_rec<T>(i, pos, vel, ri);
     } else if (k == W.K) {  // the cell's list is full: its members are found by scanning cell_of
       atomicOr((unsigned long long *)&W.st->status, (unsigned long long)CD_STATUS_SLOTS_FULL);
     }
@@ -1315,6 +1298,27 @@ __device__ __forceinline__ Self<T> self_of(const Agents<T> &A, int i, double2 po
   return s;
 }
 
+// Wall contacts of an agent from the binned walls: only the segments listed
+// for the agent's wall cell (a superset of those within its reach; outside
+// the grid, none).  Lane q of the agent's L takes every L-th.
+template <typename T, class Add>
+__device__ __forceinline__ void binned_walls(const FusedArgs &fa, const ScnDesc &d, int model,
+                                             int q, int L, double2 pos, V2<T> vel,
+                                             const WallSelf<T> &self, Add &&add) {
+  const double qx = (pos.x - fa.wall_minx) / fa.wall_cell;
+  const double qy = (pos.y - fa.wall_miny) / fa.wall_cell;
+  if (!(qx >= 0.0 && qy >= 0.0 && qx < (double)fa.wall_nx && qy < (double)fa.wall_ny)) return;
+  const int c = (int)qx * fa.wall_ny + (int)qy;
+  const int k0 = fa.wall_cells[c], k1 = fa.wall_cells[c + 1];
+  const int *ids = fa.wall_cells + (fa.wall_nx * fa.wall_ny + 1);
+  for (int k = k0 + q; k < k1; k += L) {
+    const double4 sg = fa.segs[d.w0 + ids[k]];
+    const double4 bx = make_double4(fmin(sg.x, sg.z), fmin(sg.y, sg.w), fmax(sg.x, sg.z),
+                                    fmax(sg.y, sg.w));
+    walls_each(self, model, pos, vel, &sg, nullptr, 1, add, 0, 1, &bx);
+  }
+}
+
 // Wall contacts of an agent served by L lanes (fused step): lane q of the
 // group takes every L-th of the walls from q, add(force x, force y, torque)
 // for each contact.  Every lane of the block calls this (have = false for
@@ -1325,23 +1329,7 @@ __device__ __forceinline__ void agent_walls(const FusedArgs &fa, const ScnDesc &
                                             int model, int q, int L, bool have, double2 pos,
                                             V2<T> vel, const WallSelf<T> &self, Add &&add) {
   if (fa.wall_cells) {
-    // binned walls: only the segments listed for the agent's wall cell
-    // (a superset of those within its reach; outside the grid, none)
-    if (have) {
-      const double qx = (pos.x - fa.wall_minx) / fa.wall_cell;
-      const double qy = (pos.y - fa.wall_miny) / fa.wall_cell;
-      if (qx >= 0.0 && qy >= 0.0 && qx < (double)fa.wall_nx && qy < (double)fa.wall_ny) {
-        const int c = (int)qx * fa.wall_ny + (int)qy;
-        const int k0 = fa.wall_cells[c], k1 = fa.wall_cells[c + 1];
-        const int *ids = fa.wall_cells + (fa.wall_nx * fa.wall_ny + 1);
-        for (int k = k0 + q; k < k1; k += L) {
-          const double4 sg = fa.segs[d.w0 + ids[k]];
-          const double4 bx = make_double4(fmin(sg.x, sg.z), fmin(sg.y, sg.w),
-                                          fmax(sg.x, sg.z), fmax(sg.y, sg.w));
-          walls_each(self, model, pos, vel, &sg, nullptr, 1, add, 0, 1, &bx);
-        }
-      }
-    }
+    if (have) binned_walls(fa, d, model, q, L, pos, vel, self, add);
     return;
   }
   const int nw = d.w1 - d.w0;
@@ -1408,30 +1396,14 @@ __device__ __forceinline__ void agent_forces(const FusedArgs &fa, const ScnDesc 
   if (MODEL) tq += ps.m.value();
 }
 
-// What a wave of the direct kernel keeps in LDS: the queue of candidates
-// that passed the gate (slot or agent, and which of the wave's agents they
-// belong to), the agents' side of their pairs, and the agents' exact sums.
-// A sum is a Fix128 in three limbs (weights 2^-64, 2^-32 and 1, each
-// 64-bit, the last signed), so a term joins it by plain integer atomics
-// with no carry between them; limbs hold 2^32 terms.
-constexpr int kWaveAgents = 32;  // agents of a wave at 2 lanes each
-
-template <typename T, int MODEL>
-struct WaveLds {
-  static constexpr int U = sizeof(T) == 8 ? 2 : 4;  // candidates gated per lane and round
-  static constexpr int kQueue = 64 * (U + 1);       // fewer than 64 stay between rounds
-  static constexpr int NC = MODEL ? 3 : 2;          // force x, y (and torque)
-  int slot[kQueue];
-  int own[kQueue];
-  unsigned long long lo[NC][kWaveAgents], mid[NC][kWaveAgents], hi[NC][kWaveAgents];
-  int bad[NC][kWaveAgents];
-  T neg_mk[kWaveAgents], tau_0[kWaveAgents], mu[kWaveAgents], kappa[kWaveAgents],
-      damping[kWaveAgents], rtau_0[kWaveAgents];
-  double2 pos[MODEL ? 1 : kWaveAgents];
-  V2<T> vel[MODEL ? 1 : kWaveAgents];
-  double r[MODEL ? 1 : kWaveAgents];
-  int id[MODEL ? kWaveAgents : 1];
-
+// The exact sums of the agents a wave serves, in LDS.  A sum is a Fix128 in
+// three limbs (weights 2^-64, 2^-32 and 1, each 64-bit, the last signed), so
+// a term joins it by plain integer atomics with no carry between them; limbs
+// hold 2^32 terms.
+template <int NC, int AGENTS>  // force x, y (and torque)
+struct WaveSums {
+  unsigned long long lo[NC][AGENTS], mid[NC][AGENTS], hi[NC][AGENTS];
+  int bad[NC][AGENTS];
   __device__ __forceinline__ void clear(int g) {
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
@@ -1448,8 +1420,8 @@ struct WaveLds {
     auto put = [](unsigned long long *p, unsigned long long x) {
       __hip_atomic_fetch_add(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
-    if (sizeof(X) == 8) put(&lo[c][g], t.lo & 0xffffffffull);
-    else if ((t.lo & 0xffffffffull) != 0ull) put(&lo[c][g], t.lo & 0xffffffffull);
+    // (a float's grid leaves the lowest limb alone)
+    if (sizeof(X) == 8 || (t.lo & 0xffffffffull) != 0ull) put(&lo[c][g], t.lo & 0xffffffffull);
     put(&mid[c][g], t.lo >> 32);
     put(&hi[c][g], (unsigned long long)t.hi);
   }
@@ -1460,6 +1432,31 @@ struct WaveLds {
     t.bad = bad[c][g] != 0;
     return t.value();
   }
+};
+
+// What a wave of the direct kernel keeps in LDS: the queue of candidates
+// that passed the gate (and which of the wave's agents they belong to), the
+// agents' side of their pairs, and the agents' sums.
+constexpr int kWaveAgents = 32;  // agents of a wave at 2 lanes each
+
+template <typename T, int MODEL>
+struct WaveLds {
+  static constexpr int U = sizeof(T) == 8 ? 2 : 4;  // candidates gated per lane and round
+  static constexpr int kQueue = 64 * (U + 1);       // fewer than 64 stay between rounds
+  union {
+    struct {
+      int cand[kQueue], own[kQueue];
+    };
+    unsigned long long red[8 * kWaveAgents];  // the agents' reductions, after the queue
+  };
+  WaveSums<MODEL ? 3 : 2, kWaveAgents> sum;
+  T neg_mk[kWaveAgents], tau_0[kWaveAgents], mu[kWaveAgents], kappa[kWaveAgents],
+      damping[kWaveAgents], rtau_0[kWaveAgents];
+  double2 pos[MODEL ? 1 : kWaveAgents];
+  V2<T> vel[MODEL ? 1 : kWaveAgents];
+  double r[MODEL ? 1 : kWaveAgents];
+  int id[MODEL ? kWaveAgents : 1];
+
   __device__ __forceinline__ Owner<T> owner(int g) const {
     Owner<T> o;
     o.neg_mk = neg_mk[g];
@@ -1479,6 +1476,16 @@ __device__ __forceinline__ void wave_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// body_reach of a neighbour.
+template <typename T, int MODEL>
+__device__ __forceinline__ double nbr_reach(const Agents<T> &A, const Nbr<T> &N, int j,
+                                            double2 xj) {
+  if constexpr (MODEL == 0)
+    return A.radius[j];
+  else
+    return tc_reach(xj, N.ls[j], N.rs[j], A.r_t[j], A.r_s[j]);
+}
+
 // Pair terms of a wave's agents (L lanes each), into the wave's sums.  Every
 // lane calls this (on = false for idle lanes and without a valid binning).
 //
@@ -1495,12 +1502,13 @@ __device__ __forceinline__ void wave_fence() {
 // candidates at cells of sight + 2 r, a fifth at 0.6 m.  Evaluating pairs
 // where they were met, a wave ran the pair function (300 instructions in
 // fp64) for nearly every candidate of its busiest lane.
-template <typename T, int MODEL, bool FUSED>
+template <typename T, int MODEL>
 __device__ __forceinline__ void wave_pairs(const Agents<T> &A, const Work &W, const Nbr<T> &N,
-                                           const int *count, const NbrRec<T> *rec,
-                                           const ScnDesc &d, int nx, int ny, int L, bool on,
-                                           int i, int c, int self_slot, double2 pos, V2<T> vel,
-                                           double ri, WaveLds<T, MODEL> &S) {
+                                           const int *count, const ScnDesc &d, int nx, int ny,
+                                           int L, bool on, int i, int c, double2 pos, V2<T> vel,
+                                           double reach, WaveLds<T, MODEL> &S) {
+  const NbrRec<T> *rec = (const NbrRec<T> *)W.rec;
+  const float my_gate = gate_reach(reach);
   constexpr int U = WaveLds<T, MODEL>::U;
   const int lane = threadIdx.x & 63;
   const int lg = __builtin_ctz(L);  // L is a power of two
@@ -1510,7 +1518,6 @@ __device__ __forceinline__ void wave_pairs(const Agents<T> &A, const Work &W, co
   // members are found by scanning cell_of below).
   int pre[10], so[9];
   bool over = false;
-  int sidx = -1;  // the agent's own place among the candidates
   {
     const int lc = c - d.c0, lx = ny > 0 ? lc / ny : 0, ly = lc - lx * ny;
     int n[9];
@@ -1534,35 +1541,25 @@ __device__ __forceinline__ void wave_pairs(const Agents<T> &A, const Work &W, co
       pre[k + 1] = pre[k] + (full ? 0 : n[k]);
       so[k] -= pre[k];
     }
-    if (FUSED && on && n[4] <= W.K) sidx = pre[4] + self_slot;
   }
   const int tot = pre[9];
   int idx = q;
   int jx = over ? d.a0 + q : d.a1;
   int cnt = 0;  // candidates in the queue (the same in every lane)
-  auto push = [&](bool pass, int e) {
+  auto push = [&](bool pass, int j) {
     const unsigned long long m = __ballot(pass);
     if (pass) {
       const int at = cnt + (int)__builtin_amdgcn_mbcnt_hi(
                                (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-      S.slot[at] = e;
+      S.cand[at] = j;
       S.own[at] = g;
     }
     cnt += __popcll(m);
   };
-  auto gate = [&](double2 xj, V2<T> vj, double rj) -> bool {
-    if constexpr (MODEL == 0)
-      return pair_circular_gate<T>((T)(pos.x - xj.x), (T)(pos.y - xj.y), vel.x - vj.x,
-                                   vel.y - vj.y, (T)(ri + rj));
-    else
-      return pair_three_circle_gate<T>((T)(pos.x - xj.x), (T)(pos.y - xj.y), vel.x - vj.x,
-                                       vel.y - vj.y, (T)(ri + rj));
-  };
-  auto reach_of = [&](int j, double2 xj) -> double {
-    if constexpr (MODEL == 0)
-      return A.radius[j];
-    else
-      return tc_reach(xj, N.ls[j], N.rs[j], A.r_t[j], A.r_s[j]);
+  auto gate = [&](const NbrRec<T> &r) -> bool {
+    return r.id != i && pair_gate((float)(pos.x - r.x), (float)(pos.y - r.y),
+                                  (float)(vel.x - r.vel.x), (float)(vel.y - r.vel.y),
+                                  my_gate + r.gate);
   };
   for (;;) {
     bool last = false;
@@ -1572,7 +1569,7 @@ __device__ __forceinline__ void wave_pairs(const Agents<T> &A, const Work &W, co
       for (int u = 0; u < U; ++u) {
         const int at = idx + u * L;
         s[u] = -1;
-        if (at < tot && at != sidx) {
+        if (at < tot) {
           int o = so[0];
 #pragma unroll
           for (int k = 1; k < 9; ++k)
@@ -1581,41 +1578,17 @@ __device__ __forceinline__ void wave_pairs(const Agents<T> &A, const Work &W, co
         }
       }
       idx += U * L;
-      if constexpr (FUSED) {
-        NbrRec<T> rr[U];
+      NbrRec<T> rr[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-          if (s[u] >= 0) rr[u] = rec[s[u]];
+      for (int u = 0; u < U; ++u)
+        if (s[u] >= 0) rr[u] = rec[s[u]];
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-          push(s[u] >= 0 && gate(rr[u].pos, rr[u].vel, rr[u].r), s[u]);
-        // the batch's loads have all been consumed; waiting for them here
-        // says so to the compiler, which otherwise holds each load of the
-        // next batch until the previous one arrives
-        // (s_waitcnt vmcnt(0), expcnt and lgkmcnt left at their maxima)
-        __builtin_amdgcn_s_waitcnt(0x0F70);
-      } else {
-        int j[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          j[u] = s[u] >= 0 ? W.ell_ids[s[u]] : i;
-        }
-        double2 xj[U];
-        V2<T> vj[U];
-        double rj[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          if (s[u] >= 0) {
-            xj[u] = N.pos[j[u]];
-            vj[u] = N.vel[j[u]];
-            rj[u] = reach_of(j[u], xj[u]);
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-          push(s[u] >= 0 && j[u] != i && gate(xj[u], vj[u], rj[u]), ~j[u]);
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // as above
-      }
+      for (int u = 0; u < U; ++u) push(s[u] >= 0 && gate(rr[u]), MODEL ? rr[u].id : s[u]);
+      // the batch's loads have all been consumed; waiting for them here
+      // says so to the compiler, which otherwise holds each load of the
+      // next batch until the previous one arrives
+      // (s_waitcnt vmcnt(0), expcnt and lgkmcnt left at their maxima)
+      __builtin_amdgcn_s_waitcnt(0x0F70);
     } else if (__any(jx < d.a1)) {
       // members of overfull stencil cells: the agents of the scenario whose
       // cell is one of them
@@ -1627,11 +1600,11 @@ __device__ __forceinline__ void wave_pairs(const Agents<T> &A, const Work &W, co
           const int dx = ox - lx, dy = (l - ox * ny) - (own - lx * ny);
           if (dx >= -1 && dx <= 1 && dy >= -1 && dy <= 1) {
             const double2 xj = N.pos[jx];
-            pass = gate(xj, N.vel[jx], reach_of(jx, xj));
+            pass = gate(nbr_rec<T>(jx, xj, N.vel[jx], nbr_reach<T, MODEL>(A, N, jx, xj)));
           }
         }
       }
-      push(pass, ~jx);
+      push(pass, MODEL ? jx : ~jx);
       jx += L;
     } else {
       last = true;
@@ -1641,37 +1614,30 @@ __device__ __forceinline__ void wave_pairs(const Agents<T> &A, const Work &W, co
       cnt -= m;
       wave_fence();
       if (lane < m) {
-        const int e = S.slot[cnt + lane], o = S.own[cnt + lane];
+        const int j = S.cand[cnt + lane], o = S.own[cnt + lane];
         if constexpr (MODEL == 0) {
-          double2 xj;
-          V2<T> vj;
-          double rj;
-          if (FUSED && e >= 0) {
-            const NbrRec<T> rr = rec[e];
-            xj = rr.pos;
-            vj = rr.vel;
-            rj = rr.r;
+          NbrRec<T> n;  // of a slot, or of an agent without one
+          if (j >= 0) {
+            n = rec[j];
           } else {
-            xj = N.pos[~e];
-            vj = N.vel[~e];
-            rj = A.radius[~e];
+            n = nbr_rec<T>(~j, N.pos[~j], N.vel[~j], A.radius[~j]);
           }
           const double2 xi = S.pos[o];
           const V2<T> vi = S.vel[o];
           T px, py;
-          if (pair_circular<T>((T)(xi.x - xj.x), (T)(xi.y - xj.y), vi.x - vj.x, vi.y - vj.y,
-                               (T)(S.r[o] + rj), S.owner(o), px, py)) {
-            S.add(0, o, px);
-            S.add(1, o, py);
+          if (pair_circular<T>((T)(xi.x - n.x), (T)(xi.y - n.y), vi.x - n.vel.x,
+                               vi.y - n.vel.y, (T)(S.r[o] + n.r), S.owner(o), px, py)) {
+            S.sum.add(0, o, px);
+            S.sum.add(1, o, py);
           }
         } else {
-          const int j = e >= 0 ? W.ell_ids[e] : ~e, me = S.id[o];
+          const int io = S.id[o];
           T px, py;
           double m2;
-          if (pair_tc(me, j, tc_nbr(A, N, me), tc_nbr(A, N, j), S.owner(o), px, py, m2)) {
-            S.add(0, o, px);
-            S.add(1, o, py);
-            S.add(2, o, m2);
+          if (pair_tc(io, j, tc_nbr(A, N, io), tc_nbr(A, N, j), S.owner(o), px, py, m2)) {
+            S.sum.add(0, o, px);
+            S.sum.add(1, o, py);
+            S.sum.add(2, o, m2);
           }
         }
       }
@@ -1719,13 +1685,16 @@ __device__ __forceinline__ void agent_finish(const Agents<T> &A, const FusedArgs
   }
 }
 
-// End of a fused force kernel: each wave's reduction of the new state (held
-// by every L-th lane) joins a sub-slot of the scenario's slot for the next
-// step (no block barrier); the step is counted.
-__device__ __forceinline__ void step_end(const Work &W, int scn, int p, Red r, int L) {
-  r = wave_reduce(r, L);
+// End of the tiled force kernel: each wave's reduction of the new state
+// (held by every fourth lane) joins a sub-slot of the scenario's slot for the
+// next step (no block barrier); the step is counted.
+__device__ __forceinline__ void step_end(const Work &W, int scn, int p, const Red &r,
+                                         unsigned long long *buf) {
   const int wave = (int)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
-  if ((threadIdx.x & 63) == 0) acc_merge(acc_at(W, scn, 1 - p, wave % kAccSub), r);
+  buf += 16 * 8 * (threadIdx.x >> 6);
+  if ((threadIdx.x & 3) == 0) red_put(buf, (int)(threadIdx.x & 63) >> 2, r);
+  wave_fence();
+  red_merge(acc_at(W, scn, 1 - p, wave % kAccSub), buf, 16);
   if (blockIdx.x == 0 && threadIdx.x == 0) W.st->step += 1;
 }
 
@@ -1738,7 +1707,7 @@ __device__ __forceinline__ void step_end(const Work &W, int scn, int p, Red r, i
 // Neighbour state comes from the step's snapshot, because agents move as
 // they are integrated; without a valid binning only the walls are added.
 template <typename T, int MODEL, bool FUSED, bool ONE>
-__global__ void __launch_bounds__(256, MODEL == 0 ? 3 : 1) k_forces_direct(Agents<T> A, Work W, Batch B,
+__global__ void __launch_bounds__(256, MODEL == 0 ? 3 : 2) k_forces_direct(Agents<T> A, Work W, Batch B,
                                                        FusedArgs fa, int L, int reset,
                                                        int ordered) {
   __shared__ double4 sseg[FUSED ? 3 * kWallTile : 1];
@@ -1762,18 +1731,16 @@ __global__ void __launch_bounds__(256, MODEL == 0 ? 3 : 1) k_forces_direct(Agent
   vel.x = T(0);
   vel.y = T(0);
   int c = d.c0;
-  int self_slot = -1;
   Self<T> self;
   Tail<T> tail;
   // The agent's loads come first: they need only its index, not the
   // scenario's state, whose loads would otherwise each wait for the one
-  // before.  The cell and slot are read whatever the binning's validity
-  // and used only when it holds.
+  // before.  The cell is read whatever the binning's validity and used only
+  // when it holds.
   if (have) {
     pos = A.pos[i];
     vel = A.vel[i];
     c = W.cell_of[i];
-    if (FUSED) self_slot = W.rank[i];
     self = self_of<T, MODEL>(A, i, pos);
     if (FUSED && lead) tail = tail_of(A, i);
   }
@@ -1798,7 +1765,7 @@ __global__ void __launch_bounds__(256, MODEL == 0 ? 3 : 1) k_forces_direct(Agent
     else
       ri = tc_reach(pos, self.w.ls, self.w.rs, self.w.rt, self.w.rsr);
   }
-  if ((threadIdx.x & (L - 1)) == 0) S.clear(g);
+  if ((threadIdx.x & (L - 1)) == 0) S.sum.clear(g);
   if (lead) {
     S.neg_mk[g] = self.o.neg_mk;
     S.tau_0[g] = self.o.tau_0;
@@ -1816,16 +1783,15 @@ __global__ void __launch_bounds__(256, MODEL == 0 ? 3 : 1) k_forces_direct(Agent
   }
   wave_fence();
   if (ok)
-    wave_pairs<T, MODEL, FUSED>(A, W, FUSED ? nbr_snapshot<T>(W) : nbr_agents(A),
-                                W.count + (size_t)p * W.cap, (const NbrRec<T> *)W.rec, d, nx, ny,
-                                L, have, i, c, self_slot, pos, vel, ri, S);
+    wave_pairs<T, MODEL>(A, W, FUSED ? nbr_snapshot<T>(W) : nbr_agents(A),
+                         W.count + (size_t)p * W.cap, d, nx, ny, L, have, i, c, pos, vel, ri, S);
   if (FUSED && (fa.flags & CD_USE_OBSTACLE)) {  // wall contacts join the same exact sums
     __syncthreads();  // walls staged
     agent_walls(fa, d, sseg, MODEL, (int)threadIdx.x & (L - 1), L, have, pos, vel, self.w,
                 [&](T cx, T cy, double mm) {
-                  S.add(0, g, cx);
-                  S.add(1, g, cy);
-                  if constexpr (MODEL == 1) S.add(2, g, mm);
+                  S.sum.add(0, g, cx);
+                  S.sum.add(1, g, cy);
+                  if constexpr (MODEL == 1) S.sum.add(2, g, mm);
                 });
   }
   wave_fence();
@@ -1833,14 +1799,20 @@ __global__ void __launch_bounds__(256, MODEL == 0 ? 3 : 1) k_forces_direct(Agent
   V2<T> f = self.f;
   double tq = self.tq;
   if (lead) {
-    f.x += (T)S.value(0, g);
-    f.y += (T)S.value(1, g);
-    if constexpr (MODEL == 1) tq += S.value(2, g);
+    f.x += (T)S.sum.value(0, g);
+    f.y += (T)S.sum.value(1, g);
+    if constexpr (MODEL == 1) tq += S.sum.value(2, g);
   }
   Red r;
   r.init();
   agent_finish<T, MODEL, FUSED>(A, fa, i, lead, f, tq, pos, vel, tail, dt, reset, r);
-  if constexpr (FUSED) step_end(W, sk.x, p, r, L);
+  if constexpr (FUSED) {  // the wave's agents join the reduction the next step reads
+    const int wave = (int)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
+    if ((threadIdx.x & (L - 1)) == 0) red_put(S.red, g, r);
+    wave_fence();
+    red_merge(acc_at(W, sk.x, 1 - p, wave % kAccSub), S.red, 64 >> lg);
+    if (blockIdx.x == 0 && threadIdx.x == 0) W.st->step += 1;
+  }
 }
 
 struct TileArgs {
@@ -2025,6 +1997,7 @@ __global__ void __launch_bounds__(kTileThreads) k_forces_tiled(Agents<T> A, Work
                                                                 int reset) {
   __shared__ TileLds<T, MODEL> S;
   __shared__ double4 sseg[3 * kWallTile];
+  __shared__ unsigned long long s_red[FUSED ? 2 * kTileThreads : 1];  // 8 words per 4 lanes
   const int2 sk = B.map_t ? B.map_t[blockIdx.x] : make_int2(0, (int)blockIdx.x);
   const ScnDesc d = desc_of(B, sk.x);
   const int nb = B.map_t ? d.nt : (int)gridDim.x;
@@ -2060,7 +2033,7 @@ __global__ void __launch_bounds__(kTileThreads) k_forces_tiled(Agents<T> A, Work
   } else {
     cell_from_memory<T, MODEL, FUSED>(A, W, fa, d, 0, 0, sseg, 0, 0, cx, red, false, sk.y, nb);
   }
-  if constexpr (FUSED) step_end(W, sk.x, p, red, 4);
+  if constexpr (FUSED) step_end(W, sk.x, p, red, s_red);
 }
 
 // ---------------------------------------------------------------------------
@@ -2115,10 +2088,10 @@ void launch_forces_m(const Agents<T> &A, const Work &W, const Batch &B, const Fu
     hipLaunchKernelGGL((k_forces_direct<T, MODEL, FUSED, true>), dim3(L.blocks_e),
                        dim3(L.threads_e), 0, s, A, W, B, fa, L.lanes, reset,
                        (FUSED && W.order_every > 0) ? 1 : 0);
-  } else {
+  } else if constexpr (FUSED) {  // (the operator paths have one scenario)
     hipLaunchKernelGGL((k_forces_direct<T, MODEL, FUSED, false>), dim3(L.blocks_e),
                        dim3(L.threads_e), 0, s, A, W, B, fa, L.lanes, reset,
-                       (FUSED && W.order_every > 0) ? 1 : 0);
+                       W.order_every > 0 ? 1 : 0);
   }
 }
 
@@ -2230,7 +2203,7 @@ int do_agent_agent(const cd_agents_t *a, double cell, const cd_workspace_t *w, h
   const Launch L = single_launch(w);
   int rc;
   if ((rc = launch_reduce(A, W, B, L.blocks_f, true, s))) return rc;
-  hipLaunchKernelGGL(k_bin_insert, dim3(L.blocks_f), dim3(kBS), 0, s, (const double2 *)A.pos,
+  hipLaunchKernelGGL((k_bin_insert<T, true>), dim3(L.blocks_f), dim3(kBS), 0, s, A, (int)a->model,
                      cell, W, B, 1);
   if ((rc = check_launch())) return rc;
   FusedArgs fa;
