@@ -527,6 +527,13 @@ __device__ __forceinline__ unsigned long long *acc_at(const Work &W, int scn, in
   return W.acc + ((size_t)(scn * 2 + slot) * kAccSub + sub) * 8;
 }
 
+// Orders a wave's own LDS accesses for the compiler (the hardware keeps them
+// in order).
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // The maximum over the lanes of equal index mod 8 (every lane gets its own).
 __device__ __forceinline__ unsigned long long max_by_field(unsigned long long v) {
 #pragma unroll
