@@ -165,35 +165,29 @@ __global__ void k_adj_dt_apply(AdjScal *sc, const V2<double> *vel, AdjView J, in
 
 using D4 = Dual<4>;
 
-// Accumulates into acc[0..7] (lx.x, lx.y, lv.x, lv.y, tau_0, mu, kappa,
-// damping) the contributions of agent i's pair with j, d = (x, y, vx, vy).
-__device__ __forceinline__ void pair_vjp(double x, double y, double vx, double vy, double r_tot,
-                                         const Owner<double> &oi, const Owner<double> &oj,
-                                         double2 lfi, double2 lfj, double acc[8]) {
-  {  // i's side: derivatives along the relative state
-    const Owner<D4> o{D4(oi.neg_mk), D4(oi.tau_0), D4(oi.mu), D4(oi.kappa), D4(oi.damping)};
-    D4 fx, fy;
-    if (!pair_circular<D4>(D4::seed(x, 0), D4::seed(y, 1), D4::seed(vx, 2), D4::seed(vy, 3),
-                           D4(r_tot), o, fx, fy))
-      return;  // beyond sight: neither side contributes
+// One of the three sides of agent i's pair with j, d = (x, y, vx, vy), added
+// to acc[0..7] (lx.x, lx.y, lv.x, lv.y, tau_0, mu, kappa, damping): side 0,
+// i's force along the relative state; side 1, i's force along i's
+// parameters; side 2, j's force -f(d; p_j) along the relative state.  `o`
+// and `lf` are the owner and adjoint force of the side's agent.  The sides
+// are one piece of code whose seeds are data, so lanes of a wave that
+// evaluate different sides stay together.
+__device__ __forceinline__ void side_vjp(double x, double y, double vx, double vy, double r_tot,
+                                         const Owner<double> &o, double2 lf, int side,
+                                         double acc[8]) {
+  const bool par = side == 1;
+  const double st = par ? 0.0 : 1.0, sp = par ? 1.0 : 0.0;
+  D4 dx(x), dy(y), dvx(vx), dvy(vy);
+  dx.d[0] = dy.d[1] = dvx.d[2] = dvy.d[3] = st;
+  Owner<D4> od{D4(o.neg_mk), D4(o.tau_0), D4(o.mu), D4(o.kappa), D4(o.damping)};
+  od.tau_0.d[0] = od.mu.d[1] = od.kappa.d[2] = od.damping.d[3] = sp;
+  D4 fx, fy;
+  if (!pair_circular<D4>(dx, dy, dvx, dvy, D4(r_tot), od, fx, fy)) return;  // beyond sight
 #pragma unroll
-    for (int k = 0; k < 4; ++k) acc[k] += lfi.x * fx.d[k] + lfi.y * fy.d[k];
-  }
-  {  // i's side: derivatives along i's parameters
-    const Owner<D4> o{D4(oi.neg_mk), D4::seed(oi.tau_0, 0), D4::seed(oi.mu, 1),
-                      D4::seed(oi.kappa, 2), D4::seed(oi.damping, 3)};
-    D4 fx, fy;
-    pair_circular<D4>(D4(x), D4(y), D4(vx), D4(vy), D4(r_tot), o, fx, fy);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) acc[4 + k] += lfi.x * fx.d[k] + lfi.y * fy.d[k];
-  }
-  {  // j's side, -f(d; p_j)
-    const Owner<D4> o{D4(oj.neg_mk), D4(oj.tau_0), D4(oj.mu), D4(oj.kappa), D4(oj.damping)};
-    D4 fx, fy;
-    pair_circular<D4>(D4::seed(x, 0), D4::seed(y, 1), D4::seed(vx, 2), D4::seed(vy, 3),
-                      D4(r_tot), o, fx, fy);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) acc[k] -= lfj.x * fx.d[k] + lfj.y * fy.d[k];
+  for (int k = 0; k < 4; ++k) {
+    const double v = lf.x * fx.d[k] + lf.y * fy.d[k];
+    acc[k] += par ? 0.0 : (side == 2 ? -v : v);
+    acc[4 + k] += par ? v : 0.0;
   }
 }
 
@@ -395,26 +389,161 @@ __device__ __forceinline__ void stencil_each(const Agents<double> &A, const Work
   }
 }
 
-// Pair adjoints of agent i with part q (of L equal parts) of its stencil's
-// candidates.
-__device__ __forceinline__ void stencil_vjp(const Agents<double> &A, const Work &W,
-                                            const AdjView &J, int c0, int nx, int ny, int lx,
-                                            int ly, int q, int L, int a0, int a1, int i,
-                                            double2 xi, double2 vi, double ri,
-                                            const Owner<double> &oi, double2 lfi,
-                                            double acc[8]) {
-  stencil_each(A, W, c0, nx, ny, lx, ly, q, L, a0, a1, i,
-               [&](int j, double2 xj, double2 vj, double rj) {
-                 pair_vjp(xi.x - xj.x, xi.y - xj.y, vi.x - vj.x, vi.y - vj.y, ri + rj, oi,
-                          owner_at(A, j), lfi, J.lam_f[j], acc);
-               });
+// Per wave of k_adjoint: the candidates of its agents that passed the gate,
+// kListPerLane for each lane of an agent (a slot index, or ~j of an agent
+// without a slot).
+constexpr int kListPerLane = 4;
+constexpr int kGated = 2;  // candidates gated per lane and round
+
+// Pair adjoints of the agents a wave serves, L lanes each (every lane calls
+// this; on = false for idle lanes and without a valid binning), into each
+// lane's acc; the lanes of an agent add up to its sums.
+//
+// The lanes walk the 3 x 3 stencil with consecutive candidates on
+// consecutive lanes and test each with the forward kernel's gate
+// (pair_gate), which passes every pair whose force is not zero by a branch;
+// those are the only pairs with a derivative.  Passing candidates join their
+// agent's list in the stencil's order (cells in order, each cell in agent
+// order), and the three sides of the listed pairs are spread over the
+// agent's lanes, so which lane adds which term depends on the state alone.
+//
+// Bound by the dual-number pair function, about a thousand fp64 instructions
+// a side: at cells of sight + 2 r only 3 % of the candidates pass the gate,
+// so evaluating each candidate in sight where it was met, its three sides
+// one after the other, took a lane some twenty evaluations, now one or two
+// (4000 agents at 16 lanes: 51.8 us a step before, 16.7 now).
+__device__ __forceinline__ void wave_vjp(const Agents<double> &A, const Work &W,
+                                         const AdjView &J, const ScnDesc &d, int nx, int ny,
+                                         int L, bool on, int i, int c, double2 xi, double2 vi,
+                                         double ri, const Owner<double> &oi, double2 lfi,
+                                         int *list, double acc[8]) {
+  const int lane = threadIdx.x & 63;
+  const int lg = __builtin_ctz(L);  // L is a power of two
+  const int q = lane & (L - 1), g = lane >> lg;
+  const unsigned long long mine = (L == 64 ? ~0ull : (1ull << L) - 1ull) << (g << lg);
+  const unsigned long long below = mine & ((1ull << lane) - 1ull);
+  list += (g << lg) * kListPerLane;
+  const float my_gate = gate_reach(ri);
+  const double2 *e_vel = (const double2 *)W.e_vel;
+  int gr[3], pre[10], n[9];
+  bool over = false;
+  const int lc = c - d.c0, lx = ny > 0 ? lc / ny : 0, ly = lc - lx * ny;
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    const int ox = lx + r - 1;
+    const bool okx = on && ox >= 0 && ox < nx;
+    gr[r] = d.c0 + ox * ny + ly - 1;
+    n[3 * r] = (okx && ly - 1 >= 0) ? W.count[gr[r]] : 0;
+    n[3 * r + 1] = okx ? W.count[gr[r] + 1] : 0;
+    n[3 * r + 2] = (okx && ly + 1 < ny) ? W.count[gr[r] + 2] : 0;
+  }
+  pre[0] = 0;
+#pragma unroll
+  for (int k = 0; k < 9; ++k) {  // an overfull cell's members are found below
+    const bool full = n[k] > W.K;
+    over = over || full;
+    pre[k + 1] = pre[k] + (full ? 0 : n[k]);
+  }
+  const int tot = pre[9];
+  int idx = q;
+  int jx = over ? d.a0 + q : d.a1;
+  int cnt = 0;  // candidates in the agent's list (the same in all its lanes)
+  auto push = [&](bool pass, int e) {
+    const unsigned long long m = __ballot(pass);
+    if (pass) list[cnt + __popcll(m & below)] = e;
+    cnt += __popcll(m & mine);
+  };
+  auto gate = [&](double2 xj, double2 vj, double rj) {
+    return pair_gate((float)(xi.x - xj.x), (float)(xi.y - xj.y), (float)(vi.x - vj.x),
+                     (float)(vi.y - vj.y), my_gate + gate_reach(rj));
+  };
+  for (;;) {
+    bool last = false;
+    if (__any(idx < tot)) {
+      int e[kGated];
+      bool pass[kGated];
+#pragma unroll
+      for (int u = 0; u < kGated; ++u) {
+        const int at = idx + u * L;
+        int base = 0, cc = gr[0];
+#pragma unroll
+        for (int k = 1; k < 9; ++k) {
+          if (at >= pre[k]) {
+            base = pre[k];
+            cc = gr[k / 3] + k % 3;
+          }
+        }
+        e[u] = at < tot ? (int)((unsigned)cc * (unsigned)W.K) + (at - base) : -1;
+      }
+      idx += kGated * L;
+#pragma unroll
+      for (int u = 0; u < kGated; ++u) {
+        pass[u] = false;
+        if (e[u] >= 0)
+          pass[u] = (W.ell_ids[e[u]] != i) & (int)gate(W.e_pos[e[u]], e_vel[e[u]], W.e_r[e[u]]);
+      }
+#pragma unroll
+      for (int u = 0; u < kGated; ++u) push(pass[u], e[u]);
+    } else if (__any(jx < d.a1)) {
+      // members of overfull stencil cells: the agents of the scenario whose
+      // cell is one of them
+      bool pass = false;
+      if (jx < d.a1 && jx != i) {
+        const int gc = W.cell_of[jx];
+        if (gc >= d.c0 && W.count[gc] > W.K) {
+          const int l = gc - d.c0, ox = l / ny;
+          const int ddx = ox - lx, ddy = (l - ox * ny) - ly;
+          if (ddx >= -1 && ddx <= 1 && ddy >= -1 && ddy <= 1) {
+            const V2<double> vj = A.vel[jx];
+            pass = gate(A.pos[jx], make_double2(vj.x, vj.y), A.radius[jx]);
+          }
+        }
+      }
+      push(pass, ~jx);
+      jx += L;
+    } else {
+      last = true;
+    }
+    // a full list (a round may add kGated L more), or the end
+    if (last || __any(cnt > (kListPerLane - kGated) * L)) {
+      wave_fence();
+      for (int t = q; t < 3 * cnt; t += L) {
+        const int s = t / 3, side = t - 3 * s, e = list[s];
+        int j = ~e;
+        double2 xj, vj;
+        double rj;
+        if (e >= 0) {
+          j = W.ell_ids[e];
+          xj = W.e_pos[e];
+          vj = e_vel[e];
+          rj = W.e_r[e];
+        } else {
+          const V2<double> v = A.vel[j];
+          xj = A.pos[j];
+          vj = make_double2(v.x, v.y);
+          rj = A.radius[j];
+        }
+        Owner<double> o = oi;
+        double2 lf = lfi;
+        if (side == 2) {
+          o = owner_at(A, j);
+          lf = J.lam_f[j];
+        }
+        side_vjp(xi.x - xj.x, xi.y - xj.y, vi.x - vj.x, vi.y - vj.y, ri + rj, o, lf, side, acc);
+      }
+      wave_fence();
+      cnt = 0;
+    }
+    if (last) break;
+  }
 }
 
-// L lanes per agent (2 to 64) as in the forward force kernel: lane q
-// takes part q of the stencil's candidates; lane 0 adds the agent's own
+// L lanes per agent (2 to 64) as in the forward force kernel: the agent's
+// pairs by wave_vjp, every L-th wall from lane q; lane 0 adds the agent's own
 // (adjusting) terms and writes the results.
 __global__ void __launch_bounds__(256) k_adjoint(Agents<double> A, Work W, Batch B, AdjView J,
                                                  FusedArgs fa, int L) {
+  __shared__ int s_list[256 * kListPerLane];
   const int flags = fa.flags;
   const int2 sk = block_e_t<true>(B);  // one scenario (single_batch)
   const ScnDesc d = desc_t<true>(B, sk.x);
@@ -427,27 +556,32 @@ __global__ void __launch_bounds__(256) k_adjoint(Agents<double> A, Work W, Batch
   if (W.order_every > 0 && i < d.a1) i = W.order[i];
   const int q = threadIdx.x & (L - 1);
   const bool have = i >= d.a0 && i < d.a1;
-  const bool binned = (flags & CD_USE_AGENT_AGENT) && ss->valid && !ss->oob[0];
   double acc[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) acc[k] = 0.0;
-  double2 lfi = make_double2(0.0, 0.0);
-  if (have) lfi = J.lam_f[i];
-  if (have && binned) {
-    const double2 xi = A.pos[i];
+  // the agent's inputs, loaded together; the cell is used only where the
+  // binning holds
+  double2 lfi = make_double2(0.0, 0.0), xi = lfi, vi = lfi;
+  double ri = 0.0;
+  int c = d.c0;
+  Owner<double> oi{0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  if (have) {
+    lfi = J.lam_f[i];
+    xi = A.pos[i];
     const V2<double> v = A.vel[i];
-    const double2 vi = make_double2(v.x, v.y);
-    const int c = W.cell_of[i] - d.c0;
-    const int ny = ss->ny, nx = ss->nx;
-    const int lx = c / ny, ly = c - lx * ny;
-    stencil_vjp(A, W, J, d.c0, nx, ny, lx, ly, q, L, d.a0, d.a1, i, xi, vi, A.radius[i],
-                owner_at(A, i), lfi, acc);
+    vi = make_double2(v.x, v.y);
+    ri = A.radius[i];
+    c = W.cell_of[i];
+    oi = owner_at(A, i);
   }
+  const int valid = ss->valid, oob = ss->oob[0], nx = ss->nx, ny = ss->ny;
+  if ((flags & CD_USE_AGENT_AGENT) && valid && !oob)  // the same for the whole grid
+    wave_vjp(A, W, J, d, nx, ny, L, have, i, c, xi, vi, ri, oi, lfi,
+             s_list + ((int)threadIdx.x & ~63) * kListPerLane, acc);
   if (have && (flags & CD_USE_OBSTACLE)) {
     // wall contacts, f_w(x_i, v_i; mu_i, kappa_i, damping_i)
-    const double2 xi = A.pos[i];
-    const V2<double> v = A.vel[i];
-    const double ri = A.radius[i], mu = A.mu[i], ka = A.kappa[i], da = A.damping[i];
+    const double2 v = vi;
+    const double mu = oi.mu, ka = oi.kappa, da = oi.damping;
     wall_contacts(fa, d, xi, ri, q, L, [&](const double4 &sg, const double4 &fr) {
       D4 fx, fy;
       wall_contact_dual<4>(D4::seed(xi.x, 0), D4::seed(xi.y, 1), D4::seed(v.x, 2),
@@ -477,7 +611,7 @@ __global__ void __launch_bounds__(256) k_adjoint(Agents<double> A, Work W, Batch
     // e0 = e_k(x_k) with navigation (logic.py:149-165)
     const double s = A.mass[i] / A.tau_adj[i];
     double Je[4];
-    const V2<double> e = step_e0(A, fa, W, i, A.pos[i], Je);
+    const V2<double> e = step_e0(A, fa, W, i, xi, Je);
     lv.x -= s * lfi.x;
     lv.y -= s * lfi.y;
     g_v0 = s * (e.x * lfi.x + e.y * lfi.y);
