@@ -96,8 +96,34 @@ inline int64_t max_blocks_f(int64_t n, int64_t S) {
   return std::max<int64_t>(kSingleParts, n / kBS + S + 1);
 }
 inline int64_t max_blocks_e(int64_t n, int64_t S) { return n / kMinForceAgents + S + 1; }
-// lanes per agent of the agent-parallel force kernel (2, 4, 8, 16, 32 or 64; 0: 4)
-inline int agent_lanes(const cd_workspace_t *w) { return w->agent_lanes > 0 ? (int)w->agent_lanes : 4; }
+// Lanes per agent of the agent-parallel force kernel and the adjoint: as the
+// workspace says, or (0) by the agents and the candidates of one's stencil,
+// nine cells of the mean number of agents per cell of the capacity.
+//
+// More lanes walk the stencil in fewer rounds of dependent loads, which is
+// most of the step while the chip is not full, and cost every wave its fixed
+// part.  Up to one wave per SIMD (64 Ki lanes) a lane is free: 200 agents at
+// 3.6 m take 32.6 us a step at 4 lanes and 23.6 at 32, at 0.6 m 22.5 and
+// 24.3.  Beyond it they pay while the waves still run in one round (three
+// per SIMD) and each lane has two candidates or more: 20000 agents at 3.6 m
+// take 40.5 us at 4 lanes, 33.9 at 8 and 39.3 at 16; at 0.6 m (3 candidates)
+// 25.9, 28.0 and 33.9.  Over that, long stencils stay with 4 lanes and short
+// ones with 2: 100000 agents at 3.6 m 123 us at 2, 98 at 4 and 99 at 8;
+// 200000 agents at 0.6 m 70 at 2 and 77 at 4.
+inline int agent_lanes(const cd_workspace_t *w) {
+  if (w->agent_lanes > 0) return (int)w->agent_lanes;
+  constexpr int64_t kOnePerSimd = 64 * 1024, kOneRound = 3 * kOnePerSimd;
+  const double cand = 9.0 * (double)w->n / (double)std::max<int64_t>(w->cell_capacity, 1);
+  int L = cand >= 32.0 ? 4 : 2;
+  while (L < 64) {
+    const int64_t lanes = 2 * L * (int64_t)w->n;
+    const bool free_ = L < 32 && lanes <= kOnePerSimd;
+    const bool pays = 2.0 * L <= std::max(4.0, cand / 2.0) && lanes <= kOneRound;
+    if (!free_ && !pays) break;
+    L *= 2;
+  }
+  return L;
+}
 
 struct Layout {
   int64_t state, scn_desc, scn_state, acc, map_f, map_e, map_t, partials, tiles;
