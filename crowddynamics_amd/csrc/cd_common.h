@@ -83,7 +83,7 @@ constexpr int kAccSub = 128;          // sub-slots of a scenario's reduction slo
 constexpr int kMaxPartsPerScn = 128;  // blocks of the partial-producing kernels per scenario
 constexpr int kSingleParts = 512;     // the same for a single (unbatched) scenario
 constexpr int kAgentsPerForceBlock = 64;  // default agents per force block (256 threads)
-constexpr int kMinForceAgents = 4;  // agents per force block: 64 threads / 16 lanes
+constexpr int kMinForceAgents = 4;  // agents per force block: 64 threads / 16 lanes, 256 / 64
 constexpr int kScanThreads = 256;
 constexpr int kScanItems = 16;
 constexpr int kScanTile = kScanThreads * kScanItems;
@@ -114,8 +114,10 @@ inline int agent_lanes(const cd_workspace_t *w) {
   if (w->agent_lanes > 0) return (int)w->agent_lanes;
   constexpr int64_t kOnePerSimd = 64 * 1024, kOneRound = 3 * kOnePerSimd;
   const double cand = 9.0 * (double)w->n / (double)std::max<int64_t>(w->cell_capacity, 1);
+  // (a batch's block map holds blocks of kMinForceAgents agents or more)
+  const int most = (w->force_threads > 0 ? (int)w->force_threads : 256) / kMinForceAgents;
   int L = cand >= 32.0 ? 4 : 2;
-  while (L < 64) {
+  while (L < most) {
     const int64_t lanes = 2 * L * (int64_t)w->n;
     const bool free_ = L < 32 && lanes <= kOnePerSimd;
     const bool pays = 2.0 * L <= std::max(4.0, cand / 2.0) && lanes <= kOneRound;
