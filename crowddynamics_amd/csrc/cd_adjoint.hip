@@ -455,7 +455,7 @@ __device__ __forceinline__ void wave_vjp(const Agents<double> &A, const Work &W,
   };
   auto gate = [&](double2 xj, double2 vj, double rj) {
     return pair_gate((float)(xi.x - xj.x), (float)(xi.y - xj.y), (float)(vi.x - vj.x),
-                     (float)(vi.y - vj.y), my_gate + gate_reach(rj));
+                     (float)(vi.y - vj.y), my_gate + gate_reach(rj)) > 0.0f;
   };
   for (;;) {
     bool last = false;

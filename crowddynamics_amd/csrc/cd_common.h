@@ -76,6 +76,7 @@ struct ScnState {
   int C_clear[2];  // cells of count buffer b that its next clearing pass must zero
   int oob[2];      // an agent fell outside the grid (stale bounding box), by buffer
   int par;         // count buffer and reduction slot of the current fused step
+  float slack;     // what the records' rounding may hide from the pair gate (grid_slack)
 };
 
 constexpr int kBS = 256;              // threads per block of per-agent kernels
@@ -191,10 +192,10 @@ Layout make_layout(const cd_workspace_t *w) {
   // offsets it is built from
   L.order = take(4 * n);
   L.order_off = take(4 * cap);
-  // the force kernels' neighbour records, one per slot (NbrRec: 48 bytes in
-  // fp64, 40 in fp32); three-circle agents, which the adjoint does not
-  // serve, keep them in its neighbour arrays (56 bytes per slot from e_pos)
-  L.rec = (w->model == CD_CIRCULAR) ? take(48 * slots) : L.e_pos;
+  // the force kernels' neighbour records, one per slot (NbrRec, 24 bytes);
+  // three-circle agents, which the adjoint does not serve, keep them in its
+  // neighbour arrays (56 bytes per slot from e_pos)
+  L.rec = (w->model == CD_CIRCULAR) ? take(24 * slots) : L.e_pos;
   L.total = o;
   return L;
 }
@@ -695,6 +696,17 @@ __device__ __forceinline__ Grid grid_of(const Red &r, double cell, int cap) {
   return g;
 }
 
+// What the rounding of two records' positions and velocities may add to the
+// distance of their agents up to the time of collision, which the pair
+// functions take no later than 30 s ahead: each coordinate is within 2^-24
+// of the grid's extent, each velocity difference within 2^-23 of the largest
+// speed.  The gate's reach grows by twice that.
+__device__ __forceinline__ float grid_slack(const Red &r) {
+  const double ex = from_ord_bits(r.v[R_MAXX]) - from_ord_bits(r.v[R_MINX]);
+  const double ey = from_ord_bits(r.v[R_MAXY]) - from_ord_bits(r.v[R_MINY]);
+  return (float)((ex + ey) * 0x1p-22 + __longlong_as_double((long long)r.v[R_VMAX]) * 0x1p-17);
+}
+
 // Records a scenario's reduction and grid (one thread per scenario); `buf`:
 // the count buffer the binning fills.
 __device__ __forceinline__ void publish_grid(const Work &W, ScnState *ss, const Red &r,
@@ -712,6 +724,7 @@ __device__ __forceinline__ void publish_grid(const Work &W, ScnState *ss, const 
   ss->nx = g.nx;
   ss->ny = g.ny;
   ss->valid = g.ok ? 1 : 0;
+  ss->slack = grid_slack(r);
   ss->C = g.ok ? g.nx * g.ny : 0;
   ss->C_clear[buf] = g.ok ? g.nx * g.ny : 0;
   if (!g.ok && has_agents)  // an empty scenario has no grid and no overflow
@@ -729,30 +742,29 @@ __device__ __forceinline__ int cell_of_pos(double2 p, const Grid &g, double cell
 // K_a / K_b: per-cell slot lists
 // ---------------------------------------------------------------------------
 
-// A slot's neighbour record: what the force kernels need of a candidate,
-// written beside the slot's id by the kernel that bins it, so a candidate
-// costs one load with no id hop.  gate: gate_reach of the agent's body; r:
-// the radius of circular agents (their pair function needs no more).  48
-// bytes in fp64, 40 in fp32 (the workspace holds 48 per slot).
-template <typename T>
-struct __attribute__((aligned(sizeof(T) == 8 ? 16 : 8))) NbrRec {
-  double x, y;
-  V2<T> vel;
-  double r;
+// A slot's neighbour record: what the force kernels' gate needs of a
+// candidate, written beside the slot's id by the kernel that bins it.
+// Position from the grid's origin and velocity in float, whose rounding
+// grid_slack covers; gate: gate_reach of the agent's body.  A pair that
+// passes is evaluated from the agents' own arrays.  (Records of 48 bytes in
+// fp64 and 40 in fp32, which held the pair function's inputs, cost the gate
+// two fp64 differences and twice the reads.)
+struct __attribute__((aligned(8))) NbrRec {
+  float x, y, vx, vy, gate;
   int id;
-  float gate;
 };
-static_assert(sizeof(NbrRec<double>) == 48 && sizeof(NbrRec<float>) == 40, "NbrRec layout");
+static_assert(sizeof(NbrRec) == 24, "NbrRec layout");
 
 template <typename T>
-__device__ __forceinline__ NbrRec<T> nbr_rec(int i, double2 pos, V2<T> vel, double reach) {
-  NbrRec<T> n;
-  n.x = pos.x;
-  n.y = pos.y;
-  n.vel = vel;
-  n.r = reach;
-  n.id = i;
+__device__ __forceinline__ NbrRec nbr_rec(int i, double2 pos, V2<T> vel, double reach, double ox,
+                                          double oy) {
+  NbrRec n;
+  n.x = (float)(pos.x - ox);
+  n.y = (float)(pos.y - oy);
+  n.vx = (float)vel.x;
+  n.vy = (float)vel.y;
   n.gate = gate_reach(reach);
+  n.id = i;
   return n;
 }
 
@@ -791,8 +803,8 @@ __device__ __forceinline__ void bin_scenario(const Agents<T> &A, int model, doub
     if (k < W.K) {
       W.ell_ids[c * W.K + k] = i;
       if constexpr (REC)
-        ((NbrRec<T> *)W.rec)[(size_t)c * W.K + k] =
-            nbr_rec<T>(i, p, A.vel[i], body_reach(A, model, i, p));
+        ((NbrRec *)W.rec)[(size_t)c * W.K + k] =
+            nbr_rec<T>(i, p, A.vel[i], body_reach(A, model, i, p), g.ox, g.oy);
     } else if (k == W.K) {  // the cell's list is full: its members are found by scanning cell_of
       atomicOr((unsigned long long *)&W.st->status, (unsigned long long)CD_STATUS_SLOTS_FULL);
     }

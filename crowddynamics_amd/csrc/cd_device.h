@@ -331,8 +331,9 @@ struct Owner {
 // hypot) feeds the contact force.  Only the pairs within 2^-40 of a
 // threshold take the library hypot.
 
-// The gate of a pair: false only where the pair function (pair_circular,
-// pair_three_circle and their fp32 forms) returns false or zeros.  (x, y)
+// The gate of a pair: positive, or not only where the pair function
+// (pair_circular, pair_three_circle and their fp32 forms) returns false or
+// zeros.  (x, y)
 // and (vx, vy) are the centres' and velocities' differences in float, R the
 // sum of the agents' gate_reach.  Each agent lies in a disc about its centre;
 // a pair adds a term only if the discs touch, c = |x|^2 - R^2 < 0, or will,
@@ -349,13 +350,13 @@ struct Owner {
 //
 // min and max take the other operand for NaN: with NaN in the velocities a
 // pair passes if it touches (and NaN joins the sum there).
-__device__ __forceinline__ bool pair_gate(float x, float y, float vx, float vy, float R) {
+__device__ __forceinline__ float pair_gate(float x, float y, float vx, float vy, float R) {
   const float nb = __builtin_fmaf(x, vx, y * vy);
   const float a = __builtin_fmaf(vx, vx, vy * vy);
   const float c = __builtin_fmaf(-R, R, __builtin_fmaf(x, x, y * y));
   const float disc = __builtin_fmaf(nb, nb, -(a * c));
   const float sight = __builtin_fmaf(2.0f * float(kSightSoc), R, float(kSightSoc * kSightSoc)) - c;
-  return __builtin_fminf(sight, __builtin_fmaxf(__builtin_fminf(disc, -nb), -c)) > 0.0f;
+  return __builtin_fminf(sight, __builtin_fmaxf(__builtin_fminf(disc, -nb), -c));
 }
 __device__ __forceinline__ float gate_reach(double reach) {
   return (float)(fabs(reach) * (1.0 + 0x1p-16) + 0x1p-7);

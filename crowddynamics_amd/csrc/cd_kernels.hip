@@ -341,26 +341,20 @@ __device__ __forceinline__ WallSelf<T> wall_self(const Agents<T> &A, int model, 
 // Wall contacts of an agent at p with velocity v over segments w_begin,
 // w_begin + w_stride, ... (core/interactions.py:107-141, 169-186):
 // add(force x, force y, torque) for each contact.
-// `frm`: the segments' frames (seg_frame), or null to compute them here.
-// `box`: the segments' bounding boxes {min x, min y, max x, max y}, or null;
-// with boxes, a segment whose box lies farther than the agent's reach from
-// its centre is skipped.  Every circle of the agent is then more than 1e-6 m
-// from the segment, so the skipped contact term is exactly the zero that
+// A segment whose bounding box lies farther than the agent's reach from its
+// centre is skipped: every circle of the agent is then more than 1e-6 m from
+// the segment, so the skipped contact term is exactly the zero that
 // evaluating it would give.
 template <typename T, class Add>
 __device__ __forceinline__ void walls_each(const WallSelf<T> &me, int model, double2 p, V2<T> v,
-                                           const double4 *seg, const double4 *frm, int W,
-                                           Add &&add, int w_begin = 0, int w_stride = 1,
-                                           const double4 *box = nullptr) {
+                                           const double4 *seg, int W, Add &&add, int w_begin = 0,
+                                           int w_stride = 1) {
   for (int w = w_begin; w < W; w += w_stride) {
-    if (box) {
-      const double4 b = box[w];
-      const double dx = fmax(fmax(b.x - p.x, p.x - b.z), 0.0);
-      const double dy = fmax(fmax(b.y - p.y, p.y - b.w), 0.0);
-      if (dx * dx + dy * dy > me.reach2) continue;
-    }
     const double4 s = seg[w];
-    const double4 fr = frm ? frm[w] : seg_frame(s.x, s.y, s.z, s.w);
+    const double dx = fmax(fmax(fmin(s.x, s.z) - p.x, p.x - fmax(s.x, s.z)), 0.0);
+    const double dy = fmax(fmax(fmin(s.y, s.w) - p.y, p.y - fmax(s.y, s.w)), 0.0);
+    if (dx * dx + dy * dy > me.reach2) continue;
+    const double4 fr = seg_frame(s.x, s.y, s.z, s.w);
     double h, nx, ny, rmx = 0.0, rmy = 0.0;
     if (!model) {
       distance_circle_line(p.x, p.y, me.r, s.x, s.y, s.z, s.w, fr, h, nx, ny);
@@ -435,15 +429,12 @@ __global__ void __launch_bounds__(256) k_walls(Agents<T> A, int model, const dou
       T cx = T(0), cy = T(0);
       double m = 0.0;
       if (live && w < (unsigned)W) {
-        const double4 s = segs[w];
-        const double4 box = make_double4(fmin(s.x, s.z), fmin(s.y, s.w), fmax(s.x, s.z),
-                                         fmax(s.y, s.w));
-        walls_each(me, model, p, v, &s, nullptr, 1, [&](T x, T y, double t) {
+        walls_each(me, model, p, v, segs + w, 1, [&](T x, T y, double t) {
           hit = true;
           cx = x;
           cy = y;
           m = t;
-        }, 0, 1, &box);
+        });
       }
       // the agents' contacts, in segment order (every lane keeps the sums)
       unsigned hits = (unsigned)(__ballot(hit) >> (threadIdx.x & 63 & ~(kWallLanes - 1))) &
@@ -499,7 +490,7 @@ constexpr int kTileThreads = 256;
 constexpr int kTileGroups = kTileThreads / 4;  // agents served at once
 constexpr int kTileMaxDim = 16;
 constexpr int kRegionMax = (kTileMaxDim + 2) * (kTileMaxDim + 2);
-constexpr int kWallTile = 128;  // wall segments staged in LDS at once (12 KB with frames and boxes)
+constexpr int kWallTile = 128;  // wall segments staged in LDS at once (4 KB)
 
 // LDS capacity (agents of a region): nine cells of up to 128 (circular) or
 // 56 (three-circle) agents fit, so a 3 x 3 region fits whenever no cell
@@ -962,7 +953,7 @@ __global__ void __launch_bounds__(256) k_step_begin(Agents<T> A, Work W, Batch B
     if (c < 0) return;
     if (k < W.K) {
       W.ell_ids[c * W.K + k] = i;
-      ((NbrRec<T> *)W.rec)[(size_t)c * W.K + k] = nbr_rec<T>(i, pos, vel, ri);
+      ((NbrRec *)W.rec)[(size_t)c * W.K + k] = nbr_rec<T>(i, pos, vel, ri, g.ox, g.oy);
     } else if (k == W.K) {  // the cell's list is full: its members are found by scanning cell_of
       atomicOr((unsigned long long *)&W.st->status, (unsigned long long)CD_STATUS_SLOTS_FULL);
     }
@@ -1223,17 +1214,11 @@ struct MemRow {
   }
 };
 
-// Stages cnt wall segments, their frames (seg_frame) and bounding boxes in
-// LDS: sseg holds 3 kWallTile entries, the segments, then the frames, then
-// the boxes.
+// Stages cnt wall segments in LDS.  (Their frames and boxes, staged beside
+// them, took 8 KB of each block and a square root and two divisions before
+// the first candidate; few lanes ever need a frame.)
 __device__ __forceinline__ void stage_segs(const double4 *src, int cnt, double4 *sseg) {
-  for (int k = threadIdx.x; k < cnt; k += blockDim.x) {
-    const double4 s = src[k];
-    sseg[k] = s;
-    sseg[kWallTile + k] = seg_frame(s.x, s.y, s.z, s.w);
-    sseg[2 * kWallTile + k] =
-        make_double4(fmin(s.x, s.z), fmin(s.y, s.w), fmax(s.x, s.z), fmax(s.y, s.w));
-  }
+  for (int k = threadIdx.x; k < cnt; k += blockDim.x) sseg[k] = src[k];
 }
 
 // Stages the scenario's first kWallTile wall segments (before the per-agent
@@ -1338,10 +1323,7 @@ __device__ __forceinline__ void binned_walls(const FusedArgs &fa, const ScnDesc 
   const int k0 = fa.wall_cells[c], k1 = fa.wall_cells[c + 1];
   const int *ids = fa.wall_cells + (fa.wall_nx * fa.wall_ny + 1);
   for (int k = k0 + q; k < k1; k += L) {
-    const double4 sg = fa.segs[d.w0 + ids[k]];
-    const double4 bx = make_double4(fmin(sg.x, sg.z), fmin(sg.y, sg.w), fmax(sg.x, sg.z),
-                                    fmax(sg.y, sg.w));
-    walls_each(self, model, pos, vel, &sg, nullptr, 1, add, 0, 1, &bx);
+    walls_each(self, model, pos, vel, fa.segs + d.w0 + ids[k], 1, add);
   }
 }
 
@@ -1359,14 +1341,13 @@ __device__ __forceinline__ void agent_walls(const FusedArgs &fa, const ScnDesc &
     return;
   }
   const int nw = d.w1 - d.w0;
-  const double4 *sfrm = sseg + kWallTile, *sbox = sseg + 2 * kWallTile;
-  if (have) walls_each(self, model, pos, vel, sseg, sfrm, min(kWallTile, nw), add, q, L, sbox);
+  if (have) walls_each(self, model, pos, vel, sseg, min(kWallTile, nw), add, q, L);
   for (int w0 = kWallTile; w0 < nw; w0 += kWallTile) {  // more segments than staged
     const int cnt = min(kWallTile, nw - w0);
     __syncthreads();
     stage_segs(fa.segs + d.w0 + w0, cnt, sseg);
     __syncthreads();
-    if (have) walls_each(self, model, pos, vel, sseg, sfrm, cnt, add, q, L, sbox);
+    if (have) walls_each(self, model, pos, vel, sseg, cnt, add, q, L);
   }
   if (nw > kWallTile) {  // restore the first tile for the next agents
     __syncthreads();
@@ -1467,7 +1448,7 @@ constexpr int kWaveAgents = 32;  // agents of a wave at 2 lanes each
 
 template <typename T, int MODEL>
 struct WaveLds {
-  static constexpr int U = sizeof(T) == 8 ? 2 : 4;  // candidates gated per lane and round
+  static constexpr int U = 4;                       // candidates gated per lane and round
   static constexpr int kQueue = 64 * (U + 1);       // fewer than 64 stay between rounds
   union {
     struct {
@@ -1516,18 +1497,26 @@ __device__ __forceinline__ double nbr_reach(const Agents<T> &A, const Nbr<T> &N,
 // one of them, for whichever agent it belongs to.  The sums are exact, so
 // neither who evaluates a pair nor when changes a result.
 //
-// Bound by the instructions of the walk and the gate.  A pair in sight adds
-// a term only if the two are on a collision course or touch: 3 % of the
-// candidates at cells of sight + 2 r, a fifth at 0.6 m.  Evaluating pairs
-// where they were met, a wave ran the pair function (300 instructions in
-// fp64) for nearly every candidate of its busiest lane.
+// Bound by the instructions of the walk and the gate, some 45 a candidate,
+// of which the search for its cell is a third (256 rooms at 4 lanes: the vector
+// units 89 % busy).  A pair in sight adds a term only if the two are on a
+// collision course or touch: 3 % of the candidates at cells of sight + 2 r,
+// a fifth at 0.6 m.  Evaluating pairs where they were met, a wave ran the pair
+// function (300 instructions in fp64) for nearly every candidate of its
+// busiest lane.  256 rooms, fp32: 449 us with fp64 records and a branch
+// for each lane's end, 280 now.  Walking the three rows of cells one after
+// the other (two comparisons a candidate instead of eight) idles lanes at
+// each row's end and was slower (1835 against 1690 us for five steps), and so
+// was fetching one half of a round while the other is gated (2008).
 template <typename T, int MODEL>
 __device__ __forceinline__ void wave_pairs(const Agents<T> &A, const Work &W, const Nbr<T> &N,
                                            const int *count, const ScnDesc &d, int nx, int ny,
-                                           int L, bool on, int i, int c, double2 pos, V2<T> vel,
-                                           double reach, WaveLds<T, MODEL> &S) {
-  const NbrRec<T> *rec = (const NbrRec<T> *)W.rec;
-  const float my_gate = gate_reach(reach);
+                                           double2 origin, float slack, int L, bool on, int i,
+                                           int c, double2 pos, V2<T> vel, double reach,
+                                           WaveLds<T, MODEL> &S) {
+  const NbrRec *rec = (const NbrRec *)W.rec;
+  const NbrRec me = nbr_rec<T>(i, pos, vel, reach, origin.x, origin.y);
+  const float my_gate = me.gate + slack;
   constexpr int U = WaveLds<T, MODEL>::U;
   const int lane = threadIdx.x & 63;
   const int lg = __builtin_ctz(L);  // L is a power of two
@@ -1562,47 +1551,58 @@ __device__ __forceinline__ void wave_pairs(const Agents<T> &A, const Work &W, co
     }
   }
   const int tot = pre[9];
+  if (tot == 0) so[0] = 1;  // candidate -1 (below) in slot 0
   int idx = q;
   int jx = over ? d.a0 + q : d.a1;
   int cnt = 0;  // candidates in the queue (the same in every lane)
-  auto push = [&](bool pass, int j) {
-    const unsigned long long m = __ballot(pass);
-    if (pass) {
-      const int at = cnt + (int)__builtin_amdgcn_mbcnt_hi(
-                               (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+  auto push = [&](unsigned long long m, int j) {  // the lanes of m
+    if (__builtin_amdgcn_inverse_ballot_w64(m)) {
+      const int at = (int)__builtin_amdgcn_mbcnt_hi(
+          (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, (unsigned)cnt));
       S.cand[at] = j;
       S.own[at] = g;
     }
     cnt += __popcll(m);
   };
-  auto gate = [&](const NbrRec<T> &r) -> bool {
-    return r.id != i && pair_gate((float)(pos.x - r.x), (float)(pos.y - r.y),
-                                  (float)(vel.x - r.vel.x), (float)(vel.y - r.vel.y),
-                                  my_gate + r.gate);
+  auto gate = [&](const NbrRec &r) {
+    return pair_gate(me.x - r.x, me.y - r.y, me.vx - r.vx, me.vy - r.vy, my_gate + r.gate);
+  };
+  // One round: the next N candidates of every lane.  Lanes past their
+  // stencil's end take its last candidate again, so that nothing depends on a
+  // branch and the N searches for a candidate's cell run side by side.
+  auto round = [&](auto batch) {
+    constexpr int N = decltype(batch)::value;
+    int at[N], o[N];
+    NbrRec rr[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      at[u] = min(idx + u * L, tot - 1);
+      o[u] = so[0];
+    }
+#pragma unroll
+    for (int k = 1; k < 9; ++k)
+#pragma unroll
+      for (int u = 0; u < N; ++u) o[u] = at[u] >= pre[k] ? so[k] : o[u];
+#pragma unroll
+    for (int u = 0; u < N; ++u) rr[u] = rec[o[u] + at[u]];
+    __builtin_amdgcn_sched_barrier(0);  // all loads leave before the first is used
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      constexpr int kGt = 2, kNe = 33, kLt = 40;  // the builtins' ordered >, != and signed <
+      push(__builtin_amdgcn_fcmpf(gate(rr[u]), 0.0f, kGt) &
+               __builtin_amdgcn_sicmp(rr[u].id, i, kNe) &
+               __builtin_amdgcn_sicmp(idx + u * L, tot, kLt),
+           rr[u].id);
+    }
+    idx += N * L;
   };
   for (;;) {
     bool last = false;
     if (__any(idx < tot)) {
-      int s[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int at = idx + u * L;
-        s[u] = -1;
-        if (at < tot) {
-          int o = so[0];
-#pragma unroll
-          for (int k = 1; k < 9; ++k)
-            if (at >= pre[k]) o = so[k];
-          s[u] = o + at;
-        }
-      }
-      idx += U * L;
-      NbrRec<T> rr[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (s[u] >= 0) rr[u] = rec[s[u]];
-#pragma unroll
-      for (int u = 0; u < U; ++u) push(s[u] >= 0 && gate(rr[u]), MODEL ? rr[u].id : s[u]);
+      if (__any(idx + U / 2 * L < tot))
+        round(std::integral_constant<int, U>());
+      else
+        round(std::integral_constant<int, U / 2>());
       // the batch's loads have all been consumed; waiting for them here
       // says so to the compiler, which otherwise holds each load of the
       // next batch until the previous one arrives
@@ -1619,11 +1619,12 @@ __device__ __forceinline__ void wave_pairs(const Agents<T> &A, const Work &W, co
           const int dx = ox - lx, dy = (l - ox * ny) - (own - lx * ny);
           if (dx >= -1 && dx <= 1 && dy >= -1 && dy <= 1) {
             const double2 xj = N.pos[jx];
-            pass = gate(nbr_rec<T>(jx, xj, N.vel[jx], nbr_reach<T, MODEL>(A, N, jx, xj)));
+            pass = gate(nbr_rec<T>(jx, xj, N.vel[jx], nbr_reach<T, MODEL>(A, N, jx, xj), origin.x,
+                                   origin.y)) > 0.0f;
           }
         }
       }
-      push(pass, MODEL ? jx : ~jx);
+      push(__builtin_amdgcn_ballot_w64(pass), jx);
       jx += L;
     } else {
       last = true;
@@ -1635,17 +1636,11 @@ __device__ __forceinline__ void wave_pairs(const Agents<T> &A, const Work &W, co
       if (lane < m) {
         const int j = S.cand[cnt + lane], o = S.own[cnt + lane];
         if constexpr (MODEL == 0) {
-          NbrRec<T> n;  // of a slot, or of an agent without one
-          if (j >= 0) {
-            n = rec[j];
-          } else {
-            n = nbr_rec<T>(~j, N.pos[~j], N.vel[~j], A.radius[~j]);
-          }
-          const double2 xi = S.pos[o];
-          const V2<T> vi = S.vel[o];
+          const double2 xj = N.pos[j], xi = S.pos[o];
+          const V2<T> vj = N.vel[j], vi = S.vel[o];
           T px, py;
-          if (pair_circular<T>((T)(xi.x - n.x), (T)(xi.y - n.y), vi.x - n.vel.x,
-                               vi.y - n.vel.y, (T)(S.r[o] + n.r), S.owner(o), px, py)) {
+          if (pair_circular<T>((T)(xi.x - xj.x), (T)(xi.y - xj.y), vi.x - vj.x, vi.y - vj.y,
+                               (T)(S.r[o] + A.radius[j]), S.owner(o), px, py)) {
             S.sum.add(0, o, px);
             S.sum.add(1, o, py);
           }
@@ -1729,7 +1724,7 @@ template <typename T, int MODEL, bool FUSED, bool ONE>
 __global__ void __launch_bounds__(256, MODEL == 0 ? 3 : 2) k_forces_direct(Agents<T> A, Work W, Batch B,
                                                        FusedArgs fa, int L, int reset,
                                                        int ordered) {
-  __shared__ double4 sseg[FUSED ? 3 * kWallTile : 1];
+  __shared__ double4 sseg[FUSED ? kWallTile : 1];
   __shared__ WaveLds<T, MODEL> s_wave[4];
   const int2 sk = block_e_t<ONE>(B);
   const ScnDesc d = desc_t<ONE>(B, sk.x);
@@ -1768,6 +1763,8 @@ __global__ void __launch_bounds__(256, MODEL == 0 ? 3 : 2) k_forces_direct(Agent
   const ScnState *ss = &B.sst[sk.x];
   const int par = ss->par, valid = ss->valid, oob0 = ss->oob[0], oob1 = ss->oob[1];
   const int nx = ss->nx, ny = ss->ny;
+  const double2 origin = make_double2(ss->origin[0], ss->origin[1]);
+  const float slack = ss->slack;
   const double dt_s = ss->dt;
   const int p = FUSED ? par : 0;
   const bool pairs_on = FUSED ? ((fa.flags & CD_USE_AGENT_AGENT) != 0) : true;
@@ -1803,7 +1800,8 @@ __global__ void __launch_bounds__(256, MODEL == 0 ? 3 : 2) k_forces_direct(Agent
   wave_fence();
   if (ok)
     wave_pairs<T, MODEL>(A, W, FUSED ? nbr_snapshot<T>(W) : nbr_agents(A),
-                         W.count + (size_t)p * W.cap, d, nx, ny, L, have, i, c, pos, vel, ri, S);
+                         W.count + (size_t)p * W.cap, d, nx, ny, origin, slack, L, have, i, c, pos,
+                         vel, ri, S);
   if (FUSED && (fa.flags & CD_USE_OBSTACLE)) {  // wall contacts join the same exact sums
     __syncthreads();  // walls staged
     agent_walls(fa, d, sseg, MODEL, (int)threadIdx.x & (L - 1), L, have, pos, vel, self.w,
@@ -2015,7 +2013,7 @@ __global__ void __launch_bounds__(kTileThreads) k_forces_tiled(Agents<T> A, Work
                                                                 FusedArgs fa, TileArgs ta,
                                                                 int reset) {
   __shared__ TileLds<T, MODEL> S;
-  __shared__ double4 sseg[3 * kWallTile];
+  __shared__ double4 sseg[kWallTile];
   __shared__ unsigned long long s_red[FUSED ? 2 * kTileThreads : 1];  // 8 words per 4 lanes
   const int2 sk = B.map_t ? B.map_t[blockIdx.x] : make_int2(0, (int)blockIdx.x);
   const ScnDesc d = desc_of(B, sk.x);
