@@ -56,15 +56,42 @@ inline int64_t field_tiles(int64_t rows, int64_t cols) {
 
 enum : uint8_t { F_FREE = 0, F_FROZEN = 2, F_MASKED = 3 };
 
-__device__ __forceinline__ double eik_update(double a, double b, double h) {
-  if (a > b) {
-    const double t = a;
-    a = b;
-    b = t;
-  }
-  if (__builtin_isinf(b) || b - a >= h) return a + h;
-  const double d = a - b;
-  return (a + b + sqrt(2.0 * h * h - d * d)) / 2.0;
+// Minimum and maximum of values that are never NaN.  (The library's take a
+// canonicalising instruction for each operand, on the relaxation's chain.)
+__device__ __forceinline__ double min_num(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ double max_num(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
+// The correctly rounded square root of x in [2^-760, 2^1000]: the hardware
+// reciprocal root and Goldschmidt steps, without the scaling that sqrt adds
+// for the rest of the range.
+__device__ __forceinline__ double sqrt_mid(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = __builtin_fma(-h, g, 0.5);
+  g = __builtin_fma(g, r, g);
+  const double d0 = __builtin_fma(-g, g, x);
+  h = __builtin_fma(h, r, h);
+  g = __builtin_fma(d0, h, g);
+  const double d1 = __builtin_fma(-g, g, x);
+  return __builtin_fma(d1, h, g);
+}
+
+// The update from the smaller neighbour values a <= b along the two axes
+// (a finite), h2 = 2 h^2.
+template <bool MID>
+__device__ __forceinline__ double eik_update(double a, double b, double h, double h2) {
+  const double d = b - a;
+  const double x = h2 - d * d;
+  const double two = (a + b + (MID ? sqrt_mid(x) : sqrt(x))) / 2.0;
+  return d >= h ? a + h : two;  // (b infinite: d is)
 }
 
 // Frozen nodes (on or next to the contour), free nodes at +inf, masked
@@ -127,11 +154,18 @@ __global__ void __launch_bounds__(256) k_field_init(const double *phi, const uin
 // border (or the tile itself, when the rounds ran out).
 //
 // Bound by the front's serial chain: a sweep moves it two nodes, and half a
-// sweep is one LDS round trip and one square root.  So each thread owns one
-// node of each colour (with four nodes per thread, half of them of the
-// wrong colour, the lanes idled through the other half); a node whose
-// neighbours' minima are those of its last update skips the update; and the
-// waves meet at a barrier only every fourth sweep.  Between barriers a wave
+// sweep is one LDS round trip and one square root (605 cycles; with both
+// branches of the update selected instead of taken, minima without
+// canonicalising and a square root without scaling, and the tile read
+// together with its mark, the maps below take 1.36 ms instead of 1.65, those
+// of a 311 x 156 grid 0.67 instead of 0.80).  A visit takes some 11 rounds.
+// Against 1.30 ms on another card, shorter visits (5 rounds: 1.50), tiles of
+// 64 x 32 or 16 x 16 nodes (1.71, 1.66), the colours in arrays of their own
+// (1.35) and skipping waves with nothing new nearby (1.52) were slower.
+// Each thread owns one node of each colour (with four nodes per thread, half
+// of them of the wrong colour, the lanes idled through the other half); a
+// node whose neighbours' minima are those of its last update skips the
+// update; and the waves meet at a barrier only every fourth sweep.  Between barriers a wave
 // reads its neighbours' rows as they are at that moment: values only
 // decrease and are stored whole, so an old value is one that a later sweep
 // replaces, and a round in which no thread of the block changed a node
@@ -140,6 +174,7 @@ __global__ void __launch_bounds__(256) k_field_init(const double *phi, const uin
 // blending of a 1001 x 501 grid with 24 obstacles (host work included); all
 // tiles visited in every pass, four barriers a sweep and a wait for the
 // host after each pass took 5.8 to 6.0 ms.
+template <bool MID>
 __global__ void __launch_bounds__(kFThreads) k_field_relax(int rows, int cols, double dx,
                                                            double *u, const uint8_t *state,
                                                            FieldMarks M, int pass) {
@@ -152,14 +187,19 @@ __global__ void __launch_bounds__(kFThreads) k_field_relax(int rows, int cols, d
     M.dirty[after * M.tiles + tile] = 0;
     if (tile == 0) M.live[after] = 0;
   }
-  if (!M.live[now] || !M.dirty[now * M.tiles + tile]) return;  // the same for the whole block
+  // the mark, the tile and its nodes' states are read together
+  const int marked = M.dirty[now * M.tiles + tile];
   const int r0 = blockIdx.y * kFT, c0 = blockIdx.x * kFT;
-  for (int idx = tid; idx < kFH * kFH; idx += kFThreads) {
+  constexpr int kLoads = (kFH * kFH + kFThreads - 1) / kFThreads;
+  double v[kLoads];
+#pragma unroll
+  for (int k = 0; k < kLoads; ++k) {
+    const int idx = tid + k * kFThreads;
     const int rr = r0 - 1 + idx / kFH, cc = c0 - 1 + idx % kFH;
-    su[idx] = (rr >= 0 && rr < rows && cc >= 0 && cc < cols) ? u[(int64_t)rr * cols + cc]
-                                                             : __builtin_inf();
+    v[k] = __builtin_inf();
+    if (idx < kFH * kFH && rr >= 0 && rr < rows && cc >= 0 && cc < cols)
+      v[k] = u[(int64_t)rr * cols + cc];
   }
-  if (tid < 3) s_change[tid] = 0;
   const int lr = tid / (kFT / 2);
   int lc[2];
   bool free_[2];
@@ -171,6 +211,11 @@ __global__ void __launch_bounds__(kFThreads) k_field_relax(int rows, int cols, d
     node[colour] = (int64_t)rr * cols + cc;
     free_[colour] = rr < rows && cc < cols && state[node[colour]] == F_FREE;
   }
+  if (!marked) return;  // the same for the whole block
+#pragma unroll
+  for (int k = 0; k < kLoads; ++k)
+    if (tid + k * kFThreads < kFH * kFH) su[tid + k * kFThreads] = v[k];
+  if (tid < 3) s_change[tid] = 0;
   __syncthreads();
   double own[2], first[2], plo[2], phi[2];
 #pragma unroll
@@ -181,6 +226,7 @@ __global__ void __launch_bounds__(kFThreads) k_field_relax(int rows, int cols, d
   auto at = [&](int idx) {
     return __hip_atomic_load(&su[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   };
+  const double h2 = 2.0 * dx * dx;
   bool more = true;
   for (int it = 0; it < kFRounds && more; ++it) {
     bool ch = false;
@@ -189,13 +235,13 @@ __global__ void __launch_bounds__(kFThreads) k_field_relax(int rows, int cols, d
       for (int colour = 0; colour < 2; ++colour) {
         const int idx = (lr + 1) * kFH + lc[colour] + 1;
         if (free_[colour]) {
-          const double a = fmin(at(idx - 1), at(idx + 1));
-          const double b = fmin(at(idx - kFH), at(idx + kFH));
-          const double lo = fmin(a, b), hi = fmax(a, b);
+          const double a = min_num(at(idx - 1), at(idx + 1));
+          const double b = min_num(at(idx - kFH), at(idx + kFH));
+          const double lo = min_num(a, b), hi = max_num(a, b);
           if (lo < own[colour] && (lo != plo[colour] || hi != phi[colour])) {
             plo[colour] = lo;
             phi[colour] = hi;
-            const double w = eik_update(lo, hi, dx);
+            const double w = eik_update<MID>(lo, hi, dx, h2);
             if (w < own[colour]) {
               own[colour] = w;
               __hip_atomic_store(&su[idx], w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -372,9 +418,9 @@ int cd_distance_map(const double *phi, const uint8_t *mask, int64_t rows, int64_
                      dx, out, state, M);
   int rc = check_launch();
   if (rc) return rc;
-  // every relaxation pass moves the front across at least one tile, so the
-  // passes are bounded by the tiles a shortest path can visit
-  const int64_t max_passes = 4 * ((int64_t)tiles.x * tiles.y) + 64;
+  // every pass settles at least the next node in order of distance
+  const int64_t max_passes = n + 64;
+  auto relax = (dx >= 0x1p-370 && dx <= 0x1p490) ? k_field_relax<true> : k_field_relax<false>;
   // Passes are sent in batches, with one look at the marks after each: a
   // look waits for the stream (about 40 us), a pass without marks takes 3 us.
   // An open domain takes about as many passes as the front crosses tiles,
@@ -384,8 +430,8 @@ int cd_distance_map(const double *phi, const uint8_t *mask, int64_t rows, int64_
   for (int64_t pass = 0; pass < max_passes && h_live; batch = 8) {
     const int64_t end = std::min(max_passes, pass + batch);
     for (; pass < end; ++pass)
-      hipLaunchKernelGGL(k_field_relax, tiles, dim3(kFThreads), 0, s, (int)rows, (int)cols, dx,
-                         out, (const uint8_t *)state, M, (int)(pass % 3));
+      hipLaunchKernelGGL(relax, tiles, dim3(kFThreads), 0, s, (int)rows, (int)cols, dx, out,
+                         (const uint8_t *)state, M, (int)(pass % 3));
     if ((rc = check_launch())) return rc;
     if (hipMemcpyAsync(&h_live, M.live + pass % 3, sizeof(int), hipMemcpyDeviceToHost, s) !=
             hipSuccess ||
