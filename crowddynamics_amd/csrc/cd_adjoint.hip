@@ -112,9 +112,21 @@ __device__ __forceinline__ void note_maxima(AdjScal *sc, int i, double2 v, doubl
   if (v0 == sc->v0max) atomicMin(&sc->arg_v0, i);
 }
 
-__global__ void __launch_bounds__(256) k_adj_pre(int n, const double *mass, const double *v0,
-                                                 double dt_fixed, const double2 *pos,
-                                                 const V2<double> *vel, AdjView J) {
+// The first kernel of an adjoint step after the binning: blocks up to
+// `pre_blocks` form lF, lvt and the step's lg from the next step's adjoints,
+// the others gather the cells' neighbour data.  The two share nothing; in a
+// launch of its own each took 2 to 5 us and the gap between them (rollout of
+// 4000 agents and 20 steps: 1990 us a pass, as one launch 1890).
+__global__ void __launch_bounds__(256) k_adj_pre(Agents<double> A, Work W, double dt_fixed,
+                                                 AdjView J, unsigned pre_blocks) {
+  if (blockIdx.x >= pre_blocks) {  // uniform over the block
+    cell_gather(A, W, blockIdx.x - pre_blocks);
+    return;
+  }
+  const int n = A.n;
+  const double *mass = A.mass, *v0 = A.v0;
+  const double2 *pos = A.pos;
+  const V2<double> *vel = A.vel;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const bool adaptive = J.sc != nullptr;  // uniform
   const double dt = adaptive ? J.sc->dt : dt_fixed;
@@ -811,7 +823,7 @@ int check_diff_scope(const cd_agents_t *a, const cd_step_params_t *p, const cd_w
 
 // Binning of state k (pairs) and the reduction adaptive dt is formed from.
 int diff_prepare(const Agents<double> &A, const cd_step_params_t *p, const Work &W,
-                 const Batch &B, const Launch &L, bool adaptive, hipStream_t s) {
+                 const Batch &B, const Launch &L, bool adaptive, bool gather, hipStream_t s) {
   int rc;
   const bool pairs = (p->flags & CD_USE_AGENT_AGENT) != 0;
   if (pairs || adaptive)
@@ -820,8 +832,9 @@ int diff_prepare(const Agents<double> &A, const cd_step_params_t *p, const Work 
   if (pairs) {
     hipLaunchKernelGGL((k_bin_insert<double, false>), dim3(L.blocks_f), dim3(kBS), 0, s, A, 0,
                        p->cell_size, W, B, 1);
-    hipLaunchKernelGGL(k_cell_gather<double>, dim3(grid_for((int64_t)W.cap * 64, kBS)),
-                       dim3(kBS), 0, s, A, W);
+    if (gather)
+      hipLaunchKernelGGL(k_cell_gather<double>, dim3(grid_for((int64_t)W.cap * 64, kBS)),
+                         dim3(kBS), 0, s, A, W);
   }
   return check_launch();
 }
@@ -857,10 +870,11 @@ int cd_adjoint_step(const cd_agents_t *a, const cd_step_params_t *p, const doubl
   J.x_next = (const double2 *)adj->x_next;
   J.v_next = (const double2 *)adj->v_next;
   J.sc = adaptive ? adj_scal(W) : nullptr;
-  if ((rc = diff_prepare(A, p, W, B, L, adaptive, s))) return rc;
-  hipLaunchKernelGGL(k_adj_pre, dim3(grid_for(a->n, kBS)), dim3(kBS), 0, s, (int)a->n, A.mass,
-                     (const double *)A.v0, p->dt_max, (const double2 *)A.pos,
-                     (const V2<double> *)A.vel, J);
+  if ((rc = diff_prepare(A, p, W, B, L, adaptive, false, s))) return rc;
+  const unsigned pre = (unsigned)grid_for(a->n, kBS);
+  const unsigned cells =
+      (p->flags & CD_USE_AGENT_AGENT) ? (unsigned)grid_for((int64_t)W.cap * 64, kBS) : 0u;
+  hipLaunchKernelGGL(k_adj_pre, dim3(pre + cells), dim3(kBS), 0, s, A, W, p->dt_max, J, pre);
   hipLaunchKernelGGL(k_adjoint, dim3(L.blocks_e), dim3(L.threads_e), 0, s, A, W, B, J,
                      fused_args(p), L.lanes);
   if (adaptive)
@@ -893,7 +907,7 @@ int cd_tangent_step(const cd_agents_t *a, const cd_step_params_t *p, const cd_ta
   T.x_next = (const double2 *)tan->x_next;
   T.v_next = (const double2 *)tan->v_next;
   T.sc = adaptive ? adj_scal(W) : nullptr;
-  if ((rc = diff_prepare(A, p, W, B, L, adaptive, s))) return rc;
+  if ((rc = diff_prepare(A, p, W, B, L, adaptive, true, s))) return rc;
   hipLaunchKernelGGL(k_tangent, dim3(L.blocks_e), dim3(L.threads_e), 0, s, A, W, B, T,
                      fused_args(p), L.lanes);
   if (adaptive)

@@ -849,9 +849,9 @@ __device__ __forceinline__ void gather_slot(const Agents<T> &A, const Work &W, s
 }
 
 template <typename T>
-__global__ void __launch_bounds__(256) k_cell_gather(Agents<T> A, Work W) {
+__device__ __forceinline__ void cell_gather(const Agents<T> &A, const Work &W, unsigned block) {
   const int lane = threadIdx.x & 63;
-  const int c = (int)((blockIdx.x * (size_t)blockDim.x + threadIdx.x) >> 6);
+  const int c = (int)((block * (size_t)blockDim.x + threadIdx.x) >> 6);
   if (c >= W.cap) return;  // whole waves
   const int cnt = W.count[c];
   if (cnt == 0) return;
@@ -882,6 +882,11 @@ __global__ void __launch_bounds__(256) k_cell_gather(Agents<T> A, Work W) {
     ids[t + 1] = key;
   }
   for (int s = 0; s < cnt; ++s) gather_slot(A, W, (size_t)c * W.K + s, ids[s]);
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256) k_cell_gather(Agents<T> A, Work W) {
+  cell_gather(A, W, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
