@@ -112,15 +112,42 @@ __device__ __forceinline__ void note_maxima(AdjScal *sc, int i, double2 v, doubl
   if (v0 == sc->v0max) atomicMin(&sc->arg_v0, i);
 }
 
-// The first kernel of an adjoint step after the binning: blocks up to
-// `pre_blocks` form lF, lvt and the step's lg from the next step's adjoints,
-// the others gather the cells' neighbour data.  The two share nothing; in a
-// launch of its own each took 2 to 5 us and the gap between them (rollout of
-// 4000 agents and 20 steps: 1990 us a pass, as one launch 1890).
-__global__ void __launch_bounds__(256) k_adj_pre(Agents<double> A, Work W, double dt_fixed,
-                                                 AdjView J, unsigned pre_blocks) {
-  if (blockIdx.x >= pre_blocks) {  // uniform over the block
-    cell_gather(A, W, blockIdx.x - pre_blocks);
+// State k - 1, which the sweep bins next, for the blocks that reduce it while
+// step k is prepared, and the count buffer that binning fills.
+struct NextState {
+  const double2 *pos;
+  const V2<double> *vel;
+  int *count;  // cleared here
+  int buf;     // which of the two it is
+  unsigned blocks;
+};
+
+// The first kernel of an adjoint step after the binning.  Blocks up to
+// `pre_blocks` form lF, lvt and the step's lg from the next step's adjoints;
+// the next `next.blocks` reduce the state the sweep bins next (as k_reduce,
+// into the partials this step's binning has read) and clear the counts of
+// the step before; the others gather the cells' neighbour data.  The three
+// share nothing; in launches of their own they took 2 to 5 us each and a gap
+// (rollout of 4000 agents and 20 steps: 1990 us a pass, 1800 as one).
+__global__ void __launch_bounds__(256) k_adj_pre(Agents<double> A, Work W, ScnState *ss,
+                                                 double dt_fixed, AdjView J, unsigned pre_blocks,
+                                                 NextState next) {
+  if (blockIdx.x >= pre_blocks + next.blocks) {  // uniform over the block
+    cell_gather(A, W, blockIdx.x - pre_blocks - next.blocks);
+    return;
+  }
+  if (blockIdx.x >= pre_blocks) {
+    const unsigned b = blockIdx.x - pre_blocks;
+    const int t0 = (int)(b * blockDim.x + threadIdx.x), stride = (int)(next.blocks * blockDim.x);
+    const int clear = ss->C_clear[next.buf];
+    for (int c = t0; c < clear; c += stride) next.count[c] = 0;
+    Red r;
+    r.init();
+    for (int i = t0; i < A.n; i += stride) {
+      const V2<double> v = next.vel[i];
+      r.add_agent(next.pos[i], dhypot(v.x, v.y), A.v0[i]);
+    }
+    store_partial(W, block_reduce(r), b);
     return;
   }
   const int n = A.n;
@@ -821,17 +848,20 @@ int check_diff_scope(const cd_agents_t *a, const cd_step_params_t *p, const cd_w
   return CD_OK;
 }
 
-// Binning of state k (pairs) and the reduction adaptive dt is formed from.
+// Binning of state k (pairs) into count buffer `buf` (W.count) and the
+// reduction adaptive dt is formed from.  reduced: the partials are there and
+// the buffer is clear.
 int diff_prepare(const Agents<double> &A, const cd_step_params_t *p, const Work &W,
-                 const Batch &B, const Launch &L, bool adaptive, bool gather, hipStream_t s) {
+                 const Batch &B, const Launch &L, bool adaptive, bool gather, hipStream_t s,
+                 bool reduced = false, int buf = 0) {
   int rc;
   const bool pairs = (p->flags & CD_USE_AGENT_AGENT) != 0;
-  if (pairs || adaptive)
+  if ((pairs || adaptive) && !reduced)
     if ((rc = launch_reduce(A, W, B, L.blocks_f, true, s))) return rc;
   if (adaptive) hipLaunchKernelGGL(k_adj_dt, dim3(1), dim3(kBS), 0, s, W, B, 1);
   if (pairs) {
     hipLaunchKernelGGL((k_bin_insert<double, false>), dim3(L.blocks_f), dim3(kBS), 0, s, A, 0,
-                       p->cell_size, W, B, 1);
+                       p->cell_size, W, B, 1, buf);
     if (gather)
       hipLaunchKernelGGL(k_cell_gather<double>, dim3(grid_for((int64_t)W.cap * 64, kBS)),
                          dim3(kBS), 0, s, A, W);
@@ -839,12 +869,12 @@ int diff_prepare(const Agents<double> &A, const cd_step_params_t *p, const Work 
   return check_launch();
 }
 
-}  // namespace
-
-extern "C" {
-
-int cd_adjoint_step(const cd_agents_t *a, const cd_step_params_t *p, const double *grad_x,
-                    const cd_adjoint_t *adj, const cd_workspace_t *w, cd_stream_t stream) {
+// One step of the reverse sweep.  buf: the count buffer to bin into; reduced:
+// the step before reduced this state and cleared the buffer; prev_x, prev_v:
+// the state to reduce for the next one (or null).
+int adjoint_step(const cd_agents_t *a, const cd_step_params_t *p, const double *grad_x,
+                 const cd_adjoint_t *adj, const cd_workspace_t *w, hipStream_t s, int buf,
+                 bool reduced, const double *prev_x, const double *prev_v) {
   int rc = check_step(a, p, w);
   if (rc) return rc;
   if (!adj || (a->n > 0 && (!adj->lam_x || !adj->lam_v || !adj->lam_g || !adj->lam_f ||
@@ -852,9 +882,8 @@ int cd_adjoint_step(const cd_agents_t *a, const cd_step_params_t *p, const doubl
     return CD_ERR_ARG;
   if ((rc = check_diff_scope(a, p, w, adj->x_next, adj->v_next))) return rc;
   if (a->n == 0) return CD_OK;
-  hipStream_t s = (hipStream_t)stream;
   const Agents<double> A = typed<double>(a);
-  const Work W = carve(w);
+  Work W = carve(w);
   const Batch B = single_batch(w, (p->flags & CD_USE_OBSTACLE) ? p->n_segments : 0, p->seed,
                                p->dt_min, p->dt_max);
   const Launch L = single_launch(w);
@@ -870,17 +899,34 @@ int cd_adjoint_step(const cd_agents_t *a, const cd_step_params_t *p, const doubl
   J.x_next = (const double2 *)adj->x_next;
   J.v_next = (const double2 *)adj->v_next;
   J.sc = adaptive ? adj_scal(W) : nullptr;
-  if ((rc = diff_prepare(A, p, W, B, L, adaptive, false, s))) return rc;
+  NextState next;
+  next.pos = (const double2 *)prev_x;
+  next.vel = (const V2<double> *)prev_v;
+  next.buf = 1 - buf;
+  next.count = W.count + (size_t)next.buf * W.cap;
+  next.blocks = prev_x ? (unsigned)L.blocks_f : 0u;
+  W.count += (size_t)buf * W.cap;
+  if ((rc = diff_prepare(A, p, W, B, L, adaptive, false, s, reduced, buf))) return rc;
   const unsigned pre = (unsigned)grid_for(a->n, kBS);
   const unsigned cells =
       (p->flags & CD_USE_AGENT_AGENT) ? (unsigned)grid_for((int64_t)W.cap * 64, kBS) : 0u;
-  hipLaunchKernelGGL(k_adj_pre, dim3(pre + cells), dim3(kBS), 0, s, A, W, p->dt_max, J, pre);
+  hipLaunchKernelGGL(k_adj_pre, dim3(pre + next.blocks + cells), dim3(kBS), 0, s, A, W, B.sst,
+                     p->dt_max, J, pre, next);
   hipLaunchKernelGGL(k_adjoint, dim3(L.blocks_e), dim3(L.threads_e), 0, s, A, W, B, J,
                      fused_args(p), L.lanes);
   if (adaptive)
     hipLaunchKernelGGL(k_adj_dt_apply, dim3(1), dim3(1), 0, s, J.sc, (const V2<double> *)A.vel,
                        J, (int)a->n);
   return check_launch();
+}
+
+}  // namespace
+
+extern "C" {
+
+int cd_adjoint_step(const cd_agents_t *a, const cd_step_params_t *p, const double *grad_x,
+                    const cd_adjoint_t *adj, const cd_workspace_t *w, cd_stream_t stream) {
+  return adjoint_step(a, p, grad_x, adj, w, (hipStream_t)stream, 0, false, nullptr, nullptr);
 }
 
 int cd_tangent_step(const cd_agents_t *a, const cd_step_params_t *p, const cd_tangent_t *tan,
@@ -978,13 +1024,18 @@ int cd_adjoint_segment(const cd_agents_t *a, const cd_step_params_t *p, const cd
   // reverse sweep over the segment
   cd_agents_t view = *a;
   cd_adjoint_t step_adj = *adj;
+  // (at a fixed dt each step reduces the state the next one bins)
+  const bool chain = !adaptive && (p->flags & CD_USE_AGENT_AGENT);
   for (int64_t k = k1 - 1; k >= k0; --k) {
+    const size_t prev = (size_t)(k - 1 - k0) * n2;  // (of state k - 1, when there is one)
+    const bool more = chain && k > k0;
     view.position = tape_x + (size_t)(k - k0) * n2;
     view.velocity = tape_v + (size_t)(k - k0) * n2;
     step_adj.x_next = adaptive ? tape_x + (size_t)(k + 1 - k0) * n2 : nullptr;
     step_adj.v_next = adaptive ? tape_v + (size_t)(k + 1 - k0) * n2 : nullptr;
-    if ((rc = cd_adjoint_step(&view, p, grad_x ? grad_x + (size_t)k * n2 : nullptr, &step_adj,
-                              w, stream)))
+    if ((rc = adjoint_step(&view, p, grad_x ? grad_x + (size_t)k * n2 : nullptr, &step_adj, w, s,
+                           chain ? (int)((k1 - 1 - k) & 1) : 0, chain && k < k1 - 1,
+                           more ? tape_x + prev : nullptr, more ? tape_v + prev : nullptr)))
       return rc;
   }
   return CD_OK;

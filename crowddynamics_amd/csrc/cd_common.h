@@ -517,9 +517,9 @@ __device__ Red block_reduce(Red r) {
 // its block).  The next kernel on the stream combines a scenario's
 // partials; kernel boundaries make them visible, so producers need neither
 // fences nor atomics.
-__device__ __forceinline__ void store_partial(const Work &W, const Red &r) {
+__device__ __forceinline__ void store_partial(const Work &W, const Red &r, unsigned block) {
   if (threadIdx.x == 0)
-    for (int k = 0; k < R_COUNT; ++k) W.partials[blockIdx.x * 8 + k] = r.v[k];
+    for (int k = 0; k < R_COUNT; ++k) W.partials[block * 8 + k] = r.v[k];
 }
 
 // Consumer side: every block combines its scenario's partials.
@@ -650,7 +650,7 @@ __global__ void __launch_bounds__(256) k_reduce(Agents<T> A, Work W, Batch B, in
     r.add_agent(A.pos[i], dhypot((double)w.x, (double)w.y), A.v0[i]);
   }
   r = block_reduce(r);
-  store_partial(W, r);
+  store_partial(W, r, blockIdx.x);
   if (acc_slot >= 0 && threadIdx.x == 0)
     acc_merge(acc_at(W, sk.x, acc_slot, blockIdx.x % kAccSub), r);
   if (sk.y == 0 && threadIdx.x == 0) ss->oob[0] = 0;
@@ -779,15 +779,16 @@ __device__ __forceinline__ double body_reach(const Agents<T> &A, int model, int 
 // the agents into their cells' slot lists (slots beyond cell_slots are not
 // stored; the cell count tells).  Cell indices are global: scenario base +
 // local cell.  p0: the position of the block's first agent, loaded early.
-// REC: the slots' neighbour records too.
+// REC: the slots' neighbour records too.  buf: which count buffer W.count is.
 template <typename T, bool REC>
 __device__ __forceinline__ void bin_scenario(const Agents<T> &A, int model, double2 p0,
                                              double cell, const Work &W, const ScnDesc &d,
-                                             ScnState *ss, int2 sk, const Red &r, int binning) {
+                                             ScnState *ss, int2 sk, const Red &r, int binning,
+                                             int buf) {
   const int stride = d.nf * blockDim.x;
   const int i0 = d.a0 + sk.y * blockDim.x + threadIdx.x;
   const Grid g = grid_of(r, cell, d.ccap);
-  if (sk.y == 0 && threadIdx.x == 0) publish_grid(W, ss, r, g, binning != 0, d.a1 > d.a0, 0);
+  if (sk.y == 0 && threadIdx.x == 0) publish_grid(W, ss, r, g, binning != 0, d.a1 > d.a0, buf);
   if (!binning || !g.ok) return;
   for (int i = i0; i < d.a1; i += stride) {
     const double2 p = i == i0 ? p0 : A.pos[i];
@@ -815,14 +816,14 @@ __device__ __forceinline__ void bin_scenario(const Agents<T> &A, int model, doub
 // bin_scenario.
 template <typename T, bool REC>
 __global__ void __launch_bounds__(256) k_bin_insert(Agents<T> A, int model, double cell, Work W,
-                                                    Batch B, int binning) {
+                                                    Batch B, int binning, int buf) {
   const int2 sk = block_f(B);
   const ScnDesc d = desc_of(B, sk.x);
   ScnState *ss = &B.sst[sk.x];
   const int i0 = d.a0 + sk.y * blockDim.x + threadIdx.x;
   const double2 p0 = (binning && i0 < d.a1) ? A.pos[i0] : make_double2(0.0, 0.0);
   const Red r = reduce_partials(W, d);
-  bin_scenario<T, REC>(A, model, p0, cell, W, d, ss, sk, r, binning);
+  bin_scenario<T, REC>(A, model, p0, cell, W, d, ss, sk, r, binning, buf);
 }
 
 // K_b: one wave per cell of the workspace grid.  Orders the cell's slot list

@@ -2221,7 +2221,7 @@ int do_agent_agent(const cd_agents_t *a, double cell, const cd_workspace_t *w, h
   int rc;
   if ((rc = launch_reduce(A, W, B, L.blocks_f, true, s))) return rc;
   hipLaunchKernelGGL((k_bin_insert<T, true>), dim3(L.blocks_f), dim3(kBS), 0, s, A, (int)a->model,
-                     cell, W, B, 1);
+                     cell, W, B, 1, 0);
   if ((rc = check_launch())) return rc;
   FusedArgs fa;
   memset(&fa, 0, sizeof(fa));
