@@ -833,6 +833,32 @@ __global__ void __launch_bounds__(256) k_tan_post(int n, const double *mass, dou
   T.dg[i] = df;
 }
 
+// Copies of a state's [n, 2] fields, each from `src` to one or two places
+// (null: none).  One launch where each copy cost one, 2 us and a gap; element
+// by element, as the callers' arrays need no more than a double's alignment.
+struct StateCopy {
+  const double *src[3];
+  double *dst[3], *also[3];
+  double *zero;  // set to zero (or null)
+};
+__global__ void __launch_bounds__(256) k_copy_state(int64_t n2, StateCopy c) {
+  const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (k >= n2) return;
+#pragma unroll
+  for (int f = 0; f < 3; ++f) {
+    if (!c.src[f]) continue;
+    const double v = c.src[f][k];
+    if (c.dst[f]) c.dst[f][k] = v;
+    if (c.also[f]) c.also[f][k] = v;
+  }
+  if (c.zero) c.zero[k] = 0.0;
+}
+int copy_state(int64_t n2, const StateCopy &c, hipStream_t s) {
+  if (n2 == 0) return CD_OK;
+  hipLaunchKernelGGL(k_copy_state, dim3((unsigned)((n2 + kBS - 1) / kBS)), dim3(kBS), 0, s, n2, c);
+  return check_launch();
+}
+
 // The adjoint and tangent steps' scope: circular agents in fp64, a single
 // scenario, RESET set, any other node of the standard tree; adaptive dt
 // needs the state of step k + 1.
@@ -973,17 +999,18 @@ int cd_rollout_record(const cd_agents_t *a, const cd_step_params_t *p, const cd_
   if (steps < 0 || checkpoint < 1 || !x_out || !ck_pos || !ck_vel || !ck_fprev)
     return CD_ERR_ARG;
   hipStream_t s = (hipStream_t)stream;
-  const size_t bytes = (size_t)a->n * 16;
-  auto copy = [&](void *dst, const void *src) {
-    return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, s) == hipSuccess;
-  };
-  if (!copy(x_out, a->position)) return CD_ERR_HIP;
+  const int64_t n2 = a->n * 2;
+  if (steps == 0)
+    return copy_state(n2, {{(const double *)a->position}, {x_out}, {nullptr}, nullptr}, s);
   for (int64_t k = 0; k < steps; ++k) {
     if (k % checkpoint == 0) {
-      const size_t c = (size_t)(k / checkpoint) * a->n * 2;
-      if (!copy(ck_pos + c, a->position) || !copy(ck_vel + c, a->velocity) ||
-          !copy(ck_fprev + c, a->force_prev))
-        return CD_ERR_HIP;
+      const size_t c = (size_t)(k / checkpoint) * n2;
+      const StateCopy sc = {{(const double *)a->position, (const double *)a->velocity,
+                             (const double *)a->force_prev},
+                            {ck_pos + c, ck_vel + c, ck_fprev + c},
+                            {k == 0 ? x_out : nullptr, nullptr, nullptr},
+                            nullptr};
+      if ((rc = copy_state(n2, sc, s))) return rc;
     }
     if ((rc = cd_step_tape(a, p, w, x_out + (size_t)(k + 1) * a->n * 2, nullptr, stream)))
       return rc;
@@ -1001,21 +1028,19 @@ int cd_adjoint_segment(const cd_agents_t *a, const cd_step_params_t *p, const cd
   if (k0 < 0 || k1 <= k0 || !ck_pos || !ck_vel || !ck_fprev || !tape_x || !tape_v || !adj)
     return CD_ERR_ARG;
   hipStream_t s = (hipStream_t)stream;
-  const size_t n2 = (size_t)a->n * 2, bytes = n2 * 8;
-  auto copy = [&](void *dst, const void *src) {
-    return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, s) == hipSuccess;
-  };
-  // restore the checkpoint state (force is zero after Reset)
-  if (!copy(a->position, ck_pos) || !copy(a->velocity, ck_vel) ||
-      !copy(a->force_prev, ck_fprev))
-    return CD_ERR_HIP;
-  if ((rc = cd_reset(a, stream))) return rc;
+  const size_t n2 = (size_t)a->n * 2;
+  // restore the checkpoint state (force is zero after Reset), the first of
+  // the tape
+  const StateCopy sc = {{ck_pos, ck_vel, ck_fprev},
+                        {(double *)a->position, (double *)a->velocity, (double *)a->force_prev},
+                        {tape_x, tape_v, nullptr},
+                        (double *)a->force};
+  if ((rc = copy_state((int64_t)n2, sc, s))) return rc;
   if ((rc = cd_step_prepare(a, p, w, (uint64_t)k0, stream))) return rc;
   // the states k0 .. k1 - 1 of the segment (and k1 with adaptive dt, whose
   // derivative needs the state after each step)
   const bool adaptive = p->dt_min < p->dt_max;
   const int64_t last = adaptive ? k1 : k1 - 1;
-  if (!copy(tape_x, a->position) || !copy(tape_v, a->velocity)) return CD_ERR_HIP;
   for (int64_t k = k0; k < last; ++k) {
     if ((rc = cd_step_tape(a, p, w, tape_x + (size_t)(k + 1 - k0) * n2,
                            tape_v + (size_t)(k + 1 - k0) * n2, stream)))
