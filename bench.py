@@ -78,23 +78,22 @@ def step_begin_bytes(n, cells, real_bytes=8):
     potential values of the bilinear navigation lookup 32, force, velocity
     and target direction (2 reals each); write force and target direction
     (2 reals each).  For the force kernel: write the snapshot (position 16,
-    velocity 2 reals) and the slot's neighbour record (position 16, velocity
-    2 reals, radius 8, read 8).  156 + 14 reals = 268 B/agent in fp64,
-    212 B in fp32; plus clearing the previous step's cell counts, 4 B per
-    grid cell."""
-    return n * (36 + 40 + 32 + 16 + 32 + 14 * real_bytes) + 4 * cells
+    velocity 2 reals) and the slot's neighbour record (24, radius read 8).
+    156 + 12 reals = 252 B/agent in fp64, 204 B in fp32; plus clearing the
+    previous step's cell counts, 4 B per grid cell."""
+    return n * (36 + 40 + 32 + 16 + 32 + 12 * real_bytes) + 4 * cells
 
 
 def forces_bytes(n, real_bytes=8):
     """Force kernel with the integrator (circular, fused), per agent: read
     position 16, cell index and own slot 4 + 4, radius, mass and the five
     pair and contact parameters 56, target speed 8, velocity, force and
-    previous force (2 reals each), and once as a neighbour its record
-    (position 16, velocity 2 reals, radius 8); write position 16, velocity,
-    previous force and the reset force (2 reals each).  128 + 14 reals =
-    240 B/agent in fp64, 184 B in fp32 (neighbour data counted once: every
+    previous force (2 reals each), and once as a neighbour its record 24
+    and its position 16, velocity 2 reals and radius 8; write position 16,
+    velocity, previous force and the reset force (2 reals each).  152 + 14 reals =
+    264 B/agent in fp64, 208 B in fp32 (neighbour data counted once: every
     agent is read as a neighbour from cache)."""
-    return n * (16 + 8 + 56 + 8 + 16 + 8 + 16 + 14 * real_bytes)
+    return n * (16 + 8 + 56 + 8 + 24 + 16 + 8 + 16 + 14 * real_bytes)
 
 
 def measured_traffic(kernel, threads):

@@ -1490,9 +1490,8 @@ __device__ __forceinline__ double nbr_reach(const Agents<T> &A, const Nbr<T> &N,
 // lane calls this (on = false for idle lanes and without a valid binning).
 //
 // The lanes of an agent walk its 3 x 3 stencil, consecutive candidates on
-// consecutive lanes, and test each one with the gate of the pair function
-// (pair_circular_gate, pair_three_circle_gate): it needs only products and
-// passes every pair that can add a term.  Those that pass join the wave's
+// consecutive lanes, and test each one with the gate (pair_gate): it needs
+// only products and passes every pair that can add a term.  Those that pass join the wave's
 // queue, and whenever 64 wait there (and at the end) every lane evaluates
 // one of them, for whichever agent it belongs to.  The sums are exact, so
 // neither who evaluates a pair nor when changes a result.
