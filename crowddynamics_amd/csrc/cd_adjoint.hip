@@ -163,7 +163,9 @@ __global__ void __launch_bounds__(256) k_adj_pre(Agents<double> A, Work W, ScnSt
     const double2 lx = J.lam_x[i], lv = J.lam_v[i], lg = J.lam_g[i];
     const double2 lvt = make_double2(lv.x + dt * lx.x, lv.y + dt * lx.y);
     const double c2 = dt * c;
-    J.lam_f[i] = make_double2(lg.x + c * lvt.x + c2 * lx.x, lg.y + c * lvt.y + c2 * lx.y);
+    const double2 lf = make_double2(lg.x + c * lvt.x + c2 * lx.x, lg.y + c * lvt.y + c2 * lx.y);
+    J.lam_f[i] = lf;
+    if (!(isfinite(lf.x) && isfinite(lf.y))) atomicOr(&adj_scal(W)->nonfinite, 1);
     J.lam_vt[i] = lvt;
     J.lam_g[i] = make_double2(c * lvt.x, c * lvt.y);
     if (adaptive && J.sc->inside) {
@@ -441,7 +443,9 @@ constexpr int kGated = 2;  // candidates gated per lane and round
 // The lanes walk the 3 x 3 stencil with consecutive candidates on
 // consecutive lanes and test each with the forward kernel's gate
 // (pair_gate), which passes every pair whose force is not zero by a branch;
-// those are the only pairs with a derivative.  Passing candidates join their
+// those are the only pairs with a derivative.  (`all`, when some lF is not
+// finite: every pair in sight counts, as a zero derivative times it is NaN.)
+// Passing candidates join their
 // agent's list in the stencil's order (cells in order, each cell in agent
 // order), and the three sides of the listed pairs are spread over the
 // agent's lanes, so which lane adds which term depends on the state alone.
@@ -455,7 +459,7 @@ __device__ __forceinline__ void wave_vjp(const Agents<double> &A, const Work &W,
                                          const AdjView &J, const ScnDesc &d, int nx, int ny,
                                          int L, bool on, int i, int c, double2 xi, double2 vi,
                                          double ri, const Owner<double> &oi, double2 lfi,
-                                         int *list, double acc[8]) {
+                                         bool all, int *list, double acc[8]) {
   const int lane = threadIdx.x & 63;
   const int lg = __builtin_ctz(L);  // L is a power of two
   const int q = lane & (L - 1), g = lane >> lg;
@@ -493,7 +497,7 @@ __device__ __forceinline__ void wave_vjp(const Agents<double> &A, const Work &W,
     cnt += __popcll(m & mine);
   };
   auto gate = [&](double2 xj, double2 vj, double rj) {
-    return pair_gate((float)(xi.x - xj.x), (float)(xi.y - xj.y), (float)(vi.x - vj.x),
+    return all || pair_gate((float)(xi.x - xj.x), (float)(xi.y - xj.y), (float)(vi.x - vj.x),
                      (float)(vi.y - vj.y), my_gate + gate_reach(rj)) > 0.0f;
   };
   for (;;) {
@@ -616,7 +620,7 @@ __global__ void __launch_bounds__(256) k_adjoint(Agents<double> A, Work W, Batch
   const int valid = ss->valid, oob = ss->oob[0], nx = ss->nx, ny = ss->ny;
   if ((flags & CD_USE_AGENT_AGENT) && valid && !oob)  // the same for the whole grid
     wave_vjp(A, W, J, d, nx, ny, L, have, i, c, xi, vi, ri, oi, lfi,
-             s_list + ((int)threadIdx.x & ~63) * kListPerLane, acc);
+             adj_scal(W)->nonfinite != 0, s_list + ((int)threadIdx.x & ~63) * kListPerLane, acc);
   if (have && (flags & CD_USE_OBSTACLE)) {
     // wall contacts, f_w(x_i, v_i; mu_i, kappa_i, damping_i)
     const double2 v = vi;

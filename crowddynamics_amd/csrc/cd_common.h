@@ -277,12 +277,14 @@ struct Work {
 // from (core/integrator.py:29-97), whether dt lies between its clamps (its
 // derivative is then not zero), the lowest agent index attaining each
 // maximum, the exact sum of dL/d(dt) over the agents (adjoint, as a 128-bit
-// fixed-point pair) and the tangent of dt (tangent step).
+// fixed-point pair) and the tangent of dt (tangent step).  nonfinite (also at
+// a fixed dt): an agent's lF is not finite, reset by the step's binning.
 struct AdjScal {
   double dt, vmax, v0max, ddt;
   int inside, arg_v, arg_v0, bad;
   unsigned long long ldt_lo;
   long long ldt_hi;
+  int nonfinite;
 };
 constexpr int kAdjScalOffset = 64;
 static_assert(sizeof(DevState) <= kAdjScalOffset && kAdjScalOffset + sizeof(AdjScal) <= 256,
@@ -842,6 +844,7 @@ __global__ void __launch_bounds__(256) k_bin_insert(Agents<T> A, int model, doub
   const int i0 = d.a0 + sk.y * blockDim.x + threadIdx.x;
   const double2 p0 = (binning && i0 < d.a1) ? A.pos[i0] : make_double2(0.0, 0.0);
   const Red r = reduce_partials(W, d);
+  if (!REC && blockIdx.x == 0 && threadIdx.x == 0) adj_scal(W)->nonfinite = 0;
   bin_scenario<T, REC>(A, model, p0, cell, W, d, ss, sk, r, binning, buf);
 }
 
