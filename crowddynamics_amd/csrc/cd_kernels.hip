@@ -306,9 +306,12 @@ __global__ void __launch_bounds__(256) k_reset(Agents<T> A, int model) {
 }
 
 // Agent-side inputs of the wall contacts (loaded once per agent).  reach2:
-// the square of how far from the agent's centre its body extends (radius,
-// or shoulder offset + the larger radius for three-circle agents), plus
-// 1e-6 m; a segment farther than that from the centre cannot touch it.
+// the square of how far from the agent's centre its body extends, plus
+// 1e-6 m; a segment farther than that from the centre cannot touch it.  The
+// body of circular agents is their radius; of three-circle agents, the
+// circles where the stored shoulders put them (STORED, the node: a caller's
+// shoulders lie anywhere) or r_ts + the larger radius (the fused step, whose
+// own steps put the shoulders there, as its wall grid takes them too).
 template <typename T>
 struct WallSelf {
   double r, rt, rsr, reach2;
@@ -316,7 +319,7 @@ struct WallSelf {
   T mu, kappa, damping;
 };
 
-template <typename T>
+template <typename T, bool STORED>
 __device__ __forceinline__ WallSelf<T> wall_self(const Agents<T> &A, int model, int i, double2 p) {
   WallSelf<T> w;
   w.r = A.radius[i];
@@ -333,7 +336,9 @@ __device__ __forceinline__ WallSelf<T> wall_self(const Agents<T> &A, int model, 
   w.mu = (T)A.mu[i];
   w.kappa = (T)A.kappa[i];
   w.damping = (T)A.damping[i];
-  const double reach = (model ? A.r_ts[i] + fmax(w.rt, w.rsr) : w.r) + 1e-6;
+  double body = w.r;
+  if (model) body = STORED ? tc_reach(p, w.ls, w.rs, w.rt, w.rsr) : A.r_ts[i] + fmax(w.rt, w.rsr);
+  const double reach = body + 1e-6;
   w.reach2 = reach * reach;
   return w;
 }
@@ -422,7 +427,7 @@ __global__ void __launch_bounds__(256) k_walls(Agents<T> A, int model, const dou
       v = A.vel[i];
       f = A.force[i];
       if (model) tq = A.torque[i];
-      me = wall_self(A, model, i, p);
+      me = wall_self<T, true>(A, model, i, p);
     }
     for (unsigned w = q; w - q < (unsigned)W; w += kWallLanes) {
       bool hit = false;
@@ -1303,7 +1308,7 @@ template <typename T, int MODEL>
 __device__ __forceinline__ Self<T> self_of(const Agents<T> &A, int i, double2 pos) {
   Self<T> s;
   s.o = owner_of(A, i);
-  s.w = wall_self(A, MODEL, i, pos);
+  s.w = wall_self<T, false>(A, MODEL, i, pos);
   s.f = A.force[i];
   s.tq = MODEL ? A.torque[i] : 0.0;
   return s;

@@ -260,10 +260,13 @@ typedef struct cd_step_params {
 /* Host only (no device call): bins segments ([W][4] fp64, HOST memory) into
  * square cells of side `cell` over their bounding box grown by `reach`, the
  * largest distance from an agent's centre at which a wall contact can occur
- * (circular: the radius; three-circle: r_ts + max(r_t, r_s)).  A cell lists
- * every segment whose bounding box lies within reach of it, so an agent in
- * the cell is within reach of no other segment, and an agent outside the grid
- * of none.  Writes into out[0 .. capacity) the offsets of the nx * ny cells
+ * (circular: the radius; three-circle: r_ts + max(r_t, r_s), the shoulders
+ * being r_ts from the centre, where every step puts them; the fused step
+ * takes no farther shoulder's wall contacts, with a grid or without, while
+ * cd_agent_obstacle takes them wherever the shoulders are stored).  A cell
+ * lists every segment whose bounding box lies within reach of it, so an agent
+ * in the cell is within reach of no other segment, and an agent outside the
+ * grid of none.  Writes into out[0 .. capacity) the offsets of the nx * ny cells
  * ([nx * ny + 1], flat index ix * ny + iy) followed by the segment indices,
  * and into *params the grid fields (wall_nx, wall_ny, wall_minx, wall_miny,
  * wall_cell; the caller sets wall_cells to the device copy of out).  Returns

@@ -50,3 +50,43 @@ def test_walls_equal_oracle(model, n, walls):
         assert_vec_close(got[f], want[f], scale, 1e-13, f)
     far = arr['position'][:, 0] > 40.0
     assert np.array_equal(got['force'][far], arr['force'][far])
+
+
+def _shoulders_anywhere(n, where):
+    """Three-circle agents in a box of 8 m whose shoulders do not lie r_ts
+    from the centre, and segments they touch only with those."""
+    rng = np.random.default_rng(n)
+    arr = empty_agents(n, 'three_circle')
+    arr['position'] = rng.uniform(0, 8, (n, 2))
+    arr['velocity'] = rng.normal(0, 1, (n, 2))
+    arr['radius'], arr['mass'], arr['inertia_rot'] = 0.25, 80.0, 4.0 * np.pi
+    arr['r_t'], arr['r_s'], arr['r_ts'] = 0.15, 0.1, 0.15
+    if where == 'away':
+        arr['position_ls'] = arr['position'] + rng.normal(0, 1.5, (n, 2))
+        arr['position_rs'] = arr['position'] + rng.normal(0, 0.1, (n, 2))
+    # ('unset': both at the origin, as empty_agents leaves them)
+    a = rng.uniform(0, 8, (150, 2))
+    segs = np.concatenate([a, a + rng.normal(0, 0.3, (150, 2))], 1)
+    segs[0] = (-0.05, -1.0, -0.05, 1.0)
+    return arr, segs
+
+
+@pytest.mark.parametrize('where', ['away', 'unset'])
+@pytest.mark.parametrize('n', [17, 200])
+def test_walls_with_shoulders_anywhere(where, n):
+    """The contacts of the stored shoulders, wherever they are."""
+    arr, segs = _shoulders_anywhere(n, where)
+    want = arr.copy()
+    with np.errstate(all='ignore'):
+        O.agent_obstacle(want, segs)
+    placed = arr.copy()
+    placed['position_ls'] = placed['position_rs'] = placed['position']
+    O.agent_obstacle(placed, segs)
+    # contacts that only the stored shoulders have
+    assert np.sum(want['force'].any(1) & ~placed['force'].any(1)) > 0
+    dev = DeviceAgents(arr.copy())
+    core.agent_obstacle(dev, core.segments_to_device(segs))
+    got = arr.copy()
+    dev.download(got)
+    for f in ('force', 'torque'):
+        assert_vec_close(got[f], want[f], np.full(n, 2e5 * len(segs)), 1e-13, f)  # as above
