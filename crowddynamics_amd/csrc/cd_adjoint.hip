@@ -447,8 +447,10 @@ constexpr int kGated = 2;  // candidates gated per lane and round
 // finite: every pair in sight counts, as a zero derivative times it is NaN.)
 // Passing candidates join their
 // agent's list in the stencil's order (cells in order, each cell in agent
-// order), and the three sides of the listed pairs are spread over the
-// agent's lanes, so which lane adds which term depends on the state alone.
+// order), and the three sides of the listed pairs go round the agent's lanes,
+// term t to lane t mod L.  t goes on counting where a list that filled up, the
+// agent's own or another's in the wave, was worked off, so which lane adds
+// which term, and in which order, depends on the state alone.
 //
 // Bound by the dual-number pair function, about a thousand fp64 instructions
 // a side: at cells of sight + 2 r only 3 % of the candidates pass the gate,
@@ -490,7 +492,8 @@ __device__ __forceinline__ void wave_vjp(const Agents<double> &A, const Work &W,
   const int tot = pre[9];
   int idx = q;
   int jx = over ? d.a0 + q : d.a1;
-  int cnt = 0;  // candidates in the agent's list (the same in all its lanes)
+  int cnt = 0;   // candidates in the agent's list (the same in all its lanes)
+  int done = 0;  // the lane its first term goes to
   auto push = [&](bool pass, int e) {
     const unsigned long long m = __ballot(pass);
     if (pass) list[cnt + __popcll(m & below)] = e;
@@ -550,7 +553,7 @@ __device__ __forceinline__ void wave_vjp(const Agents<double> &A, const Work &W,
     // a full list (a round may add kGated L more), or the end
     if (last || __any(cnt > (kListPerLane - kGated) * L)) {
       wave_fence();
-      for (int t = q; t < 3 * cnt; t += L) {
+      for (int t = (q - done) & (L - 1); t < 3 * cnt; t += L) {
         const int s = t / 3, side = t - 3 * s, e = list[s];
         int j = ~e;
         double2 xj, vj;
@@ -575,6 +578,7 @@ __device__ __forceinline__ void wave_vjp(const Agents<double> &A, const Work &W,
         side_vjp(xi.x - xj.x, xi.y - xj.y, vi.x - vj.x, vi.y - vj.y, ri + rj, o, lf, side, acc);
       }
       wave_fence();
+      done = (done + 3 * cnt) & (L - 1);
       cnt = 0;
     }
     if (last) break;

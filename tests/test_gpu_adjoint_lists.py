@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from crowddynamics_amd import examples as E
-from crowddynamics_amd.adjoint import Rollout
+from crowddynamics_amd.adjoint import Rollout, rollout_positions
 from tests import dense_reference as D
 
 pytestmark = pytest.mark.gpu
@@ -67,3 +67,27 @@ def test_step_equals_dense_autograd(n, side, cell):
         for c, t in enumerate(p):
             err = float((R.grad[:, c].cpu() - t.grad).abs().max())
             assert err <= 10 * tol * float(t.grad.abs().max()) + 1e-300, (lanes, c, err)
+
+
+@pytest.mark.filterwarnings('ignore')
+@pytest.mark.parametrize('n,side,lanes', [(150, 4.0, 2), (150, 4.0, 4), (150, 4.0, 16),
+                                          (400, 5.0, 2), (400, 3.0, 4)])
+def test_lists_that_fill_keep_the_bits(n, side, lanes):
+    """Which agents share a wave, and so when a wave works its lists off, does
+    not touch an agent's gradient: agents in index order, in cell order and in
+    the order of every third step give the same bits."""
+    arr = _crowd(n, side, n)
+    gen = torch.Generator().manual_seed(n + lanes)
+    w = torch.randn((5, n, 2), dtype=torch.float64, generator=gen).cuda()
+    out = []
+    for every in (0, 1, 3):
+        R = Rollout(arr, steps=4, dt=DT, cell_size=3.6, lanes=lanes, order_every=every,
+                    bounds=(-1.0, -1.0, side + 31.0, side + 31.0))
+        p = [torch.full((n,), c, dtype=torch.float64, device='cuda').requires_grad_(True)
+             for c in (3.0, 1.2e5, 4e4, 500.0)]
+        p.append(torch.as_tensor(np.array(arr['target_velocity']), device='cuda')
+                 .requires_grad_(True))
+        out.append(torch.autograd.grad(rollout_positions(R, *p), p, w))
+    for g in out[1:]:
+        for a, b in zip(g, out[0]):
+            assert torch.equal(a, b)
