@@ -77,6 +77,7 @@ struct ScnState {
   int oob[2];      // an agent fell outside the grid (stale bounding box), by buffer
   int par;         // count buffer and reduction slot of the current fused step
   float slack;     // what the records' rounding may hide from the pair gate (grid_slack)
+  float slow;      // and the square of the speeds, per distance, it may turn (gate_slow)
 };
 
 constexpr int kBS = 256;              // threads per block of per-agent kernels
@@ -718,14 +719,19 @@ __device__ __forceinline__ Grid grid_of(const Red &r, double cell, int cap) {
 }
 
 // What the rounding of two records' positions and velocities may add to the
-// distance of their agents up to the time of collision, which the pair
-// functions take no later than 30 s ahead: each coordinate is within 2^-24
-// of the grid's extent, each velocity difference within 2^-23 of the largest
-// speed.  The gate's reach grows by twice that.
+// distance of their agents up to 30 s ahead, as far as the circular pair
+// looks: each coordinate is within 2^-24 of the grid's extent, each velocity
+// difference within 2^-23 of the largest speed.  The gate's reach grows by
+// twice that.  (gate_slow: the three-circle pair looks farther, pair_gate.)
 __device__ __forceinline__ float grid_slack(const Red &r) {
   const double ex = from_ord_bits(r.v[R_MAXX]) - from_ord_bits(r.v[R_MINX]);
   const double ey = from_ord_bits(r.v[R_MAXY]) - from_ord_bits(r.v[R_MINY]);
   return (float)((ex + ey) * 0x1p-22 + __longlong_as_double((long long)r.v[R_VMAX]) * 0x1p-17);
+}
+
+__device__ __forceinline__ float gate_slow(const Red &r) {
+  const double vmax = __longlong_as_double((long long)r.v[R_VMAX]);
+  return (float)(vmax * vmax * 0x1p-29);
 }
 
 // Records a scenario's reduction and grid (one thread per scenario); `buf`:
@@ -746,6 +752,7 @@ __device__ __forceinline__ void publish_grid(const Work &W, ScnState *ss, const 
   ss->ny = g.ny;
   ss->valid = g.ok ? 1 : 0;
   ss->slack = grid_slack(r);
+  ss->slow = gate_slow(r);
   ss->C = g.ok ? g.nx * g.ny : 0;
   ss->C_clear[buf] = g.ok ? g.nx * g.ny : 0;
   if (!g.ok && has_agents)  // an empty scenario has no grid and no overflow

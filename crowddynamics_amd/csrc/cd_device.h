@@ -350,13 +350,25 @@ struct Owner {
 //
 // min and max take the other operand for NaN: with NaN in the velocities a
 // pair passes if it touches (and NaN joins the sum there).
-__device__ __forceinline__ float pair_gate(float x, float y, float vx, float vy, float R) {
+//
+// The circular pair looks 30 s ahead (kTauMax), the three-circle pair (LATE)
+// however far, so there a slow approach also passes where the velocities'
+// rounding, e = sqrt(2) 2^-23 of the largest speed at most, may hide a
+// collision: slow = (2^8 e)^2, and unless |v| < 2^8 e |x| the error of the
+// direction moves the closest approach by less than 2^-8 m, a quarter of the
+// margin 2 m.
+template <bool LATE = false>
+__device__ __forceinline__ float pair_gate(float x, float y, float vx, float vy, float R,
+                                           float slow = 0.0f) {
   const float nb = __builtin_fmaf(x, vx, y * vy);
   const float a = __builtin_fmaf(vx, vx, vy * vy);
-  const float c = __builtin_fmaf(-R, R, __builtin_fmaf(x, x, y * y));
+  const float d2 = __builtin_fmaf(x, x, y * y);
+  const float c = __builtin_fmaf(-R, R, d2);
   const float disc = __builtin_fmaf(nb, nb, -(a * c));
   const float sight = __builtin_fmaf(2.0f * float(kSightSoc), R, float(kSightSoc * kSightSoc)) - c;
-  return __builtin_fminf(sight, __builtin_fmaxf(__builtin_fminf(disc, -nb), -c));
+  float on_course = __builtin_fmaxf(__builtin_fminf(disc, -nb), -c);
+  if constexpr (LATE) on_course = __builtin_fmaxf(on_course, __builtin_fmaf(d2, slow, -a));
+  return __builtin_fminf(sight, on_course);
 }
 __device__ __forceinline__ float gate_reach(double reach) {
   return (float)(fabs(reach) * (1.0 + 0x1p-16) + 0x1p-7);

@@ -1515,9 +1515,9 @@ __device__ __forceinline__ double nbr_reach(const Agents<T> &A, const Nbr<T> &N,
 template <typename T, int MODEL>
 __device__ __forceinline__ void wave_pairs(const Agents<T> &A, const Work &W, const Nbr<T> &N,
                                            const int *count, const ScnDesc &d, int nx, int ny,
-                                           double2 origin, float slack, int L, bool on, int i,
-                                           int c, double2 pos, V2<T> vel, double reach,
-                                           WaveLds<T, MODEL> &S) {
+                                           double2 origin, float slack, float slow, int L,
+                                           bool on, int i, int c, double2 pos, V2<T> vel,
+                                           double reach, WaveLds<T, MODEL> &S) {
   const NbrRec *rec = (const NbrRec *)W.rec;
   const NbrRec me = nbr_rec<T>(i, pos, vel, reach, origin.x, origin.y);
   const float my_gate = me.gate + slack;
@@ -1569,7 +1569,9 @@ __device__ __forceinline__ void wave_pairs(const Agents<T> &A, const Work &W, co
     cnt += __popcll(m);
   };
   auto gate = [&](const NbrRec &r) {
-    return pair_gate(me.x - r.x, me.y - r.y, me.vx - r.vx, me.vy - r.vy, my_gate + r.gate);
+    constexpr bool kLate = MODEL == 1 && sizeof(T) == 8;  // (fp32 velocities are not rounded)
+    return pair_gate<kLate>(me.x - r.x, me.y - r.y, me.vx - r.vx, me.vy - r.vy, my_gate + r.gate,
+                            slow);
   };
   // One round: the next N candidates of every lane.  Lanes past their
   // stencil's end take its last candidate again, so that nothing depends on a
@@ -1768,7 +1770,7 @@ __global__ void __launch_bounds__(256, MODEL == 0 ? 3 : 2) k_forces_direct(Agent
   const int par = ss->par, valid = ss->valid, oob0 = ss->oob[0], oob1 = ss->oob[1];
   const int nx = ss->nx, ny = ss->ny;
   const double2 origin = make_double2(ss->origin[0], ss->origin[1]);
-  const float slack = ss->slack;
+  const float slack = ss->slack, slow = ss->slow;
   const double dt_s = ss->dt;
   const int p = FUSED ? par : 0;
   const bool pairs_on = FUSED ? ((fa.flags & CD_USE_AGENT_AGENT) != 0) : true;
@@ -1804,8 +1806,8 @@ __global__ void __launch_bounds__(256, MODEL == 0 ? 3 : 2) k_forces_direct(Agent
   wave_fence();
   if (ok)
     wave_pairs<T, MODEL>(A, W, FUSED ? nbr_snapshot<T>(W) : nbr_agents(A),
-                         W.count + (size_t)p * W.cap, d, nx, ny, origin, slack, L, have, i, c, pos,
-                         vel, ri, S);
+                         W.count + (size_t)p * W.cap, d, nx, ny, origin, slack, slow, L, have, i, c,
+                         pos, vel, ri, S);
   if (FUSED && (fa.flags & CD_USE_OBSTACLE)) {  // wall contacts join the same exact sums
     __syncthreads();  // walls staged
     agent_walls(fa, d, sseg, MODEL, (int)threadIdx.x & (L - 1), L, have, pos, vel, self.w,
