@@ -45,3 +45,44 @@ def test_neighbours_equal_oracle(n, side, sight, k, n_seg):
     assert np.array_equal(has.cpu().numpy(), wh)
     # the sums keep their order: a few roundings of unit vectors
     np.testing.assert_allclose(d.cpu().numpy(), wd, rtol=0, atol=1e-13)
+
+
+def _comb(side, gap):
+    """Horizontal walls `gap` apart: whoever is not in one's own strip is
+    hidden."""
+    y = np.arange(0.5 * gap, side, gap)
+    return np.stack([np.zeros_like(y), y, np.full_like(y, side), y], 1)
+
+
+@pytest.mark.parametrize('kind,n,side,sight,k', [
+    ('uniform', 130, 2.5, 3.0, 16),  # eight or nine candidates a lane
+    ('uniform', 700, 6.0, 5.0, 16),  # several hundred in sight
+    ('comb', 300, 4.0, 5.0, 8),      # and most of them hidden
+    ('comb', 300, 30.0, 40.0, 16),   # all in one cell
+    ('ties', 600, 6.0, 5.0, 16),     # rings of equal distances
+    ('heap', 300, 2.0, 3.0, 16),     # most agents at one place
+    ('heap', 290, 2.0, 1e-300, 3),   # whose squares vanish
+])
+def test_crowded_neighbours_equal_oracle(kind, n, side, sight, k):
+    """More candidates in sight than the lanes of an agent hold at once."""
+    rng = np.random.default_rng(n + k)
+    arr = empty_agents(n)
+    pos = rng.uniform(0, side, (n, 2))
+    if kind == 'ties':
+        pos = np.floor(pos / 0.25) * 0.25
+    if kind == 'heap':
+        pos[: 9 * n // 10] = pos[0]
+        if sight < 1e-200:
+            pos = np.floor(rng.uniform(0, 4, (n, 2))) * sight / 2
+    segs = _comb(side, side / 40) if kind == 'comb' else np.zeros((0, 4))
+    arr['position'] = pos
+    dev = DeviceAgents(arr)
+    cells = 100 if sight < 1e-200 else cell_capacity_for(side, side, sight)
+    got = S.find_nearest_neighbors(dev, sight, k, segs, Workspace(n, cells, 0, cell_slots=4))
+    want = O.nearest_neighbors(arr['position'], sight, k, segs)
+    if kind != 'heap':
+        d = np.hypot(*(pos[:, None] - pos[None]).transpose(2, 0, 1))
+        assert ((d < sight).sum(1) > 129).any()
+    if kind == 'comb':
+        assert (want[:, -1] < 0).any()  # looked through everyone in sight
+    assert np.array_equal(got.cpu().numpy(), want)
