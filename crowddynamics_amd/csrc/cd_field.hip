@@ -357,28 +357,47 @@ __global__ void __launch_bounds__(256) k_fill_nearest(const double *sx, const do
   dy_[k] = y0;
   if (!fill[k] || !(__builtin_isnan(x0) || __builtin_isnan(y0))) return;
   const int r = (int)(k / cols), c = (int)(k - (int64_t)r * cols);
-  // rings of growing distance; a ring at distance m holds no node nearer
-  // than m, so the search ends with the first ring beyond the best node
+  // First the square of half-width kNear, then, unless the best node is nearer
+  // than all outside it, the rest; of each the rows by growing distance and of
+  // a row the part inside the grid and the best distance so far, four nodes at
+  // a time so that their loads leave together.  Bound by those loads where no
+  // direction is near: 1000^2 nodes with a hole of 980^2 and reach 6 take
+  // 0.12 ms and with reach 100 15 ms (rings of growing width 0.13 and 24, every
+  // node of the square in turn 0.12 and 19), 100 x 100 nodes with no direction
+  // and reach 1000 0.70 ms (rings, beyond the grid too, 134; in turn 1.0).  The
+  // grown obstacles of a 1001 x 501 grid take 17 us (rings 17; in turn 52).
+  constexpr int kNear = 4;
   int best = 0x7fffffff;
   int64_t bj = -1;
-  auto look = [&](int rr, int cc) {
-    if (rr < 0 || rr >= rows || cc < 0 || cc >= cols) return;
-    const int64_t j = (int64_t)rr * cols + cc;
-    const int d2 = (rr - r) * (rr - r) + (cc - c) * (cc - c);
-    if (d2 > best || (d2 == best && j > bj)) return;  // row-major order among equals
-    if (__builtin_isnan(sx[j]) || __builtin_isnan(sy[j])) return;
-    best = d2;
-    bj = j;
+  auto scan = [&](int dr, int lo, int hi) {  // columns lo to hi of row r + dr
+    const int64_t row = (int64_t)(r + dr) * cols;
+    for (int cc = lo; cc <= hi; cc += 4) {
+      double v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = sx[row + min(cc + u, hi)];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int64_t j = row + min(cc + u, hi);
+        const int dc = min(cc + u, hi) - c, d2 = dr * dr + dc * dc;
+        if (__builtin_isnan(v[u]) || d2 > best || (d2 == best && j >= bj)) continue;
+        if (__builtin_isnan(sy[j])) continue;  // (row-major order among equals)
+        best = d2;
+        bj = j;
+      }
+    }
   };
-  for (int m = 1; m <= reach && m * m <= best; ++m) {
-    for (int t = -m; t <= m; ++t) {
-      look(r - m, c + t);
-      look(r + m, c + t);
+  for (int h = min(kNear, reach), done = -1;; done = h, h = reach) {  // done: its half-width
+    const int last = min(h, max(r, rows - 1 - r));
+    for (int m = 0; m <= last && m * m <= best; ++m) {
+      const int w = best == 0x7fffffff ? h : min(h, (int)sqrtf((float)(best - m * m)) + 1);
+      const int c0 = max(c - w, 0), c1 = min(c + w, cols - 1);
+      for (int dr = -m; dr <= m; dr += max(2 * m, 1)) {
+        if (r + dr < 0 || r + dr >= rows) continue;
+        scan(dr, c0, m <= done ? c - done - 1 : c1);
+        if (m <= done) scan(dr, c + done + 1, c1);
+      }
     }
-    for (int t = -m + 1; t < m; ++t) {
-      look(r + t, c - m);
-      look(r + t, c + m);
-    }
+    if (h == reach || best < (h + 1) * (h + 1)) break;
   }
   if (bj >= 0) {
     dx_[k] = sx[bj];

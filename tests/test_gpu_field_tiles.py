@@ -68,3 +68,32 @@ def test_fill_takes_the_first_of_the_nearest(reach):
             wx[r, c], wy[r, c] = ex[rr[k] + r0, cc[k] + c0], ey[rr[k] + r0, cc[k] + c0]
     assert np.array_equal(ox.cpu().numpy(), wx, equal_nan=True)
     assert np.array_equal(oy.cpu().numpy(), wy, equal_nan=True)
+
+
+@pytest.mark.parametrize('rows,cols,every,reach', [
+    (37, 41, 0, 1024),   # no direction anywhere, squares far beyond the grid
+    (37, 41, 13, 1024),  # few, whose distances tie
+    (3, 300, 90, 200),
+    (300, 3, 90, 200),
+    (40, 60, 12, 5),     # nodes with none within reach beside ones with four
+    (40, 60, 9, 8),
+])
+def test_fill_reaches_past_the_nearest_square(rows, cols, every, reach):
+    ex = np.full((rows, cols), np.nan)
+    if every:
+        at = ex[every // 3::every, every // 3::every]
+        at[...] = 1.0 + np.arange(at.size).reshape(at.shape)
+        ex[0, -1] = -1.0
+    fb = F.FieldBuilder(_grid(rows, cols))
+    t = torch.as_tensor(ex, device='cuda')
+    ox, oy = fb.fill_missing(t, 2.0 * t, np.ones((rows, cols), dtype=bool), reach)
+    have = np.argwhere(~np.isnan(ex))  # row-major
+    want = ex.copy()
+    for r, c in np.argwhere(np.isnan(ex)):
+        d = have - (r, c)
+        near = (np.abs(d) <= reach).all(1)
+        if near.any():
+            k = np.flatnonzero(near)[np.argmin((d[near] ** 2).sum(1))]
+            want[r, c] = ex[tuple(have[k])]
+    assert np.array_equal(ox.cpu().numpy(), want, equal_nan=True)
+    assert np.array_equal(oy.cpu().numpy(), 2.0 * want, equal_nan=True)
