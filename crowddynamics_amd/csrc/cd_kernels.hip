@@ -406,16 +406,24 @@ __device__ __forceinline__ void walls_each(const WallSelf<T> &me, int model, dou
 // about one segment in all; the few contacts are then added one after the
 // other in segment order.  One thread per agent evaluating each segment took
 // 42 us for 2000 three-circle agents and 16 segments, this 4.2 us.
+//
+// Where the agents alone fill the chip, the lanes of one repeat its loads and
+// its sums: one lane an agent for few segments.  us a call at 16, 2 and 1
+// lanes, three-circle: 200000 agents, 4 segments 32, 9 and 9, 64 segments 47,
+// 30 and 26; 1000000 agents, 4 segments 146, 31 and 28 (without the box test
+// 29), 64 segments 217, 117 and 96; but 100000 agents, 200 segments 45 and 47
+// at 16 and 2, 30000 agents 18 and 33.
 constexpr int kWallLanes = 16;
+constexpr int64_t kWallFullAgents = 64 * 1024, kWallFewSegments = 64;
 constexpr int kWallBlocks = 1 << 20;  // blocks stride over more agents than that holds
 
-template <typename T>
+template <typename T, int LANES>
 __global__ void __launch_bounds__(256) k_walls(Agents<T> A, int model, const double4 *segs,
                                                int W) {
-  const int q = threadIdx.x & (kWallLanes - 1);
-  const int per = (int)blockDim.x / kWallLanes;
+  const int q = threadIdx.x & (LANES - 1);
+  const int per = (int)blockDim.x / LANES;
   for (int base = blockIdx.x * per; base < A.n; base += gridDim.x * per) {
-    const int i = base + (int)threadIdx.x / kWallLanes;
+    const int i = base + (int)threadIdx.x / LANES;
     const bool live = i < A.n;
     double2 p = make_double2(0.0, 0.0);
     V2<T> v, f;
@@ -429,7 +437,7 @@ __global__ void __launch_bounds__(256) k_walls(Agents<T> A, int model, const dou
       if (model) tq = A.torque[i];
       me = wall_self<T, true>(A, model, i, p);
     }
-    for (unsigned w = q; w - q < (unsigned)W; w += kWallLanes) {
+    for (unsigned w = q; w - q < (unsigned)W; w += LANES) {
       bool hit = false;
       T cx = T(0), cy = T(0);
       double m = 0.0;
@@ -442,12 +450,12 @@ __global__ void __launch_bounds__(256) k_walls(Agents<T> A, int model, const dou
         });
       }
       // the agents' contacts, in segment order (every lane keeps the sums)
-      unsigned hits = (unsigned)(__ballot(hit) >> (threadIdx.x & 63 & ~(kWallLanes - 1))) &
-                      ((1u << kWallLanes) - 1u);
+      unsigned hits = (unsigned)(__ballot(hit) >> (threadIdx.x & 63 & ~(LANES - 1))) &
+                      ((1u << LANES) - 1u);
       while (__any(hits != 0)) {
         const int from = hits ? __builtin_ctz(hits) : 0;
-        const T ax = __shfl(cx, from, kWallLanes), ay = __shfl(cy, from, kWallLanes);
-        const double am = __shfl(m, from, kWallLanes);
+        const T ax = __shfl(cx, from, LANES), ay = __shfl(cy, from, LANES);
+        const double am = __shfl(m, from, LANES);
         if (hits) {
           f.x += ax;
           f.y += ay;
@@ -2502,12 +2510,17 @@ int cd_agent_obstacle(const cd_agents_t *a, const double *segments, int64_t W,
   if (W < 0 || (W > 0 && !segments) || W > 0x7fffffff) return CD_ERR_ARG;
   if (a->n == 0 || W == 0) return CD_OK;
   hipStream_t s = (hipStream_t)stream;
+  const bool full = a->n > kWallFullAgents && W <= kWallFewSegments;
+  const int per = kBS / (full ? 1 : kWallLanes);
+  const dim3 grid(std::min(grid_for(a->n, per), kWallBlocks));
+  auto launch = [&](auto kernel, const auto &A) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kBS), 0, s, A, (int)a->model, (const double4 *)segments,
+                       (int)W);
+  };
   if (a->real == CD_F64)
-    hipLaunchKernelGGL(k_walls<double>, dim3(std::min(grid_for(a->n, kBS / kWallLanes), kWallBlocks)), dim3(kBS), 0, s,
-                       typed<double>(a), (int)a->model, (const double4 *)segments, (int)W);
+    launch(full ? k_walls<double, 1> : k_walls<double, kWallLanes>, typed<double>(a));
   else
-    hipLaunchKernelGGL(k_walls<float>, dim3(std::min(grid_for(a->n, kBS / kWallLanes), kWallBlocks)), dim3(kBS), 0, s,
-                       typed<float>(a), (int)a->model, (const double4 *)segments, (int)W);
+    launch(full ? k_walls<float, 1> : k_walls<float, kWallLanes>, typed<float>(a));
   return check_launch();
 }
 

@@ -90,3 +90,38 @@ def test_walls_with_shoulders_anywhere(where, n):
     dev.download(got)
     for f in ('force', 'torque'):
         assert_vec_close(got[f], want[f], np.full(n, 2e5 * len(segs)), 1e-13, f)  # as above
+
+
+@pytest.mark.parametrize('model', ['circular', 'three_circle'])
+@pytest.mark.parametrize('precision', ['f64', 'f32'])
+@pytest.mark.parametrize('n,walls', [(65537, 1), (65537, 64), (65537, 65), (70001, 17)])
+def test_walls_of_a_large_crowd(model, precision, n, walls):
+    """One lane an agent beyond 65536 agents and up to 64 segments: the same
+    bits as the sixteen that serve the same agents in small groups."""
+    rng = np.random.default_rng(n + walls)
+    arr = empty_agents(n, model)
+    arr['position'] = rng.uniform(0, 20, (n, 2))
+    arr['velocity'] = rng.normal(0, 1, (n, 2)).astype(np.float32)
+    arr['force'] = rng.normal(0, 100, (n, 2)).astype(np.float32)
+    arr['radius'], arr['mass'] = rng.uniform(0.2, 0.3, n), 80.0
+    if model == 'three_circle':
+        arr['r_t'], arr['r_s'], arr['r_ts'] = 0.15, 0.1, 0.15
+        off = rng.normal(0, 0.15, (n, 2))
+        arr['position_ls'], arr['position_rs'] = arr['position'] - off, arr['position'] + off
+        arr['torque'] = rng.normal(0, 10, n)
+    segs = core.segments_to_device(rng.uniform(0, 20, (walls, 4)))
+    fields = ('force', 'torque') if model == 'three_circle' else ('force',)
+
+    def node(part):
+        dev = DeviceAgents(part.copy(), precision=precision)
+        core.agent_obstacle(dev, segs)
+        out = part.copy()
+        dev.download(out)
+        return out
+
+    got = node(arr)
+    assert np.sum((got['force'] != arr['force']).any(1)) > n // 100
+    for part in (slice(0, 5000), slice(n - 4001, n)):
+        want = node(arr[part])
+        for f in fields:
+            assert np.array_equal(got[f][part], want[f]), f
