@@ -603,9 +603,16 @@ template <typename T>
 struct Nbr {
   const double2 *pos;
   const V2<T> *vel;
+  const double *r;
+  const NbrState<T> *state;  // circular agents' snapshot in fp32, in the three's place
+  bool packed;               // whether it is (known to the compiler wherever a Nbr is used)
   const double2 *ls, *rs;
   const double *phi;    // the agent arrays' orientation (operator path) ...
   const double2 *off;   // ... or the snapshot's shoulder offsets (fused step)
+  __device__ __forceinline__ NbrState<T> circular(int j) const {
+    if (packed) return state[j];
+    return NbrState<T>{pos[j], vel[j], r[j]};
+  }
 };
 
 template <typename T>
@@ -613,6 +620,9 @@ __host__ __device__ __forceinline__ Nbr<T> nbr_agents(const Agents<T> &A) {
   Nbr<T> N;
   N.pos = A.pos;
   N.vel = A.vel;
+  N.r = A.radius;
+  N.state = nullptr;
+  N.packed = false;
   N.ls = A.ls;
   N.rs = A.rs;
   N.phi = A.phi;
@@ -621,10 +631,13 @@ __host__ __device__ __forceinline__ Nbr<T> nbr_agents(const Agents<T> &A) {
 }
 
 template <typename T>
-__host__ __device__ __forceinline__ Nbr<T> nbr_snapshot(const Work &W) {
+__host__ __device__ __forceinline__ Nbr<T> nbr_snapshot(const Agents<T> &A, const Work &W) {
   Nbr<T> N;
   N.pos = W.snap_pos;
   N.vel = (const V2<T> *)W.snap_vel;
+  N.r = A.radius;
+  N.state = (const NbrState<T> *)W.snap_pos;
+  N.packed = sizeof(T) == 4;
   N.ls = W.snap_ls;
   N.rs = W.snap_rs;
   N.phi = nullptr;
@@ -929,12 +942,14 @@ __global__ void __launch_bounds__(256) k_step_begin(Agents<T> A, Work W, Batch B
   const bool bin = binning && g.ok;
   // steps that rebuild the force kernel's processing order keep the slot ranks
   const bool ranks = W.order_every > 0 && step % (uint64_t)W.order_every == 0ull;
-  V2<T> *snap_vel = (V2<T> *)W.snap_vel;
   // an agent's snapshot and slot atomic (bin_begin), then its slot list
   // entry and neighbour record (bin_end)
   auto bin_begin = [&](int i, double2 pos, V2<T> vel, int &c, int &k, double &ri) {
-    W.snap_pos[i] = pos;
-    snap_vel[i] = vel;
+    constexpr bool kPacked = MODEL == 0 && sizeof(T) == 4;
+    if (!kPacked) {
+      W.snap_pos[i] = pos;
+      ((V2<T> *)W.snap_vel)[i] = vel;
+    }
     if (MODEL) {
       const double2 ls = A.ls[i], rs = A.rs[i];
       ri = bin ? tc_reach(pos, ls, rs, A.r_t[i], A.r_s[i]) : 0.0;
@@ -944,6 +959,7 @@ __global__ void __launch_bounds__(256) k_step_begin(Agents<T> A, Work W, Batch B
     } else {
       ri = bin ? A.radius[i] : 0.0;
     }
+    if (kPacked) ((NbrState<T> *)W.snap_pos)[i] = NbrState<T>{pos, vel, ri};
     c = -1;
     k = 0;
     if (bin) {
@@ -1107,10 +1123,12 @@ struct MemRow {
   template <class F>
   __device__ __forceinline__ void visit(int self, int j, F &fn) const {
     if (j == self) return;
-    if constexpr (MODEL == 0)
-      fn(j, N.pos[j], N.vel[j], A.radius[j]);
-    else
+    if constexpr (MODEL == 0) {
+      const NbrState<T> o = N.circular(j);
+      fn(j, o.pos, o.vel, o.r);
+    } else {
       fn(j, tc_nbr(A, N, j));
+    }
   }
   // The nine counts are loaded together.  A part's candidates are walked
   // in batches of four whose id and data loads are issued together, so a
@@ -1173,9 +1191,10 @@ struct MemRow {
 #pragma unroll
           for (int u = 0; u < kIdBatch; ++u) {
             if (j[u] >= 0) {
-              xj[u] = N.pos[j[u]];
-              vj[u] = N.vel[j[u]];
-              rj[u] = A.radius[j[u]];
+              const NbrState<T> o = N.circular(j[u]);
+              xj[u] = o.pos;
+              vj[u] = o.vel;
+              rj[u] = o.r;
             }
           }
 #pragma unroll
@@ -1489,16 +1508,6 @@ struct WaveLds {
   }
 };
 
-// body_reach of a neighbour.
-template <typename T, int MODEL>
-__device__ __forceinline__ double nbr_reach(const Agents<T> &A, const Nbr<T> &N, int j,
-                                            double2 xj) {
-  if constexpr (MODEL == 0)
-    return A.radius[j];
-  else
-    return tc_reach(xj, N.ls[j], N.rs[j], A.r_t[j], A.r_s[j]);
-}
-
 // Pair terms of a wave's agents (L lanes each), into the wave's sums.  Every
 // lane calls this (on = false for idle lanes and without a valid binning).
 //
@@ -1632,9 +1641,17 @@ __device__ __forceinline__ void wave_pairs(const Agents<T> &A, const Work &W, co
           const int l = gc - d.c0, ox = l / ny, own = c - d.c0, lx = own / ny;
           const int dx = ox - lx, dy = (l - ox * ny) - (own - lx * ny);
           if (dx >= -1 && dx <= 1 && dy >= -1 && dy <= 1) {
-            const double2 xj = N.pos[jx];
-            pass = gate(nbr_rec<T>(jx, xj, N.vel[jx], nbr_reach<T, MODEL>(A, N, jx, xj), origin.x,
-                                   origin.y)) > 0.0f;
+            NbrRec rj;
+            if constexpr (MODEL == 0) {
+              const NbrState<T> o = N.circular(jx);
+              rj = nbr_rec<T>(jx, o.pos, o.vel, o.r, origin.x, origin.y);
+            } else {
+              const double2 xj = N.pos[jx];
+              rj = nbr_rec<T>(jx, xj, N.vel[jx],
+                              tc_reach(xj, N.ls[jx], N.rs[jx], A.r_t[jx], A.r_s[jx]), origin.x,
+                              origin.y);
+            }
+            pass = gate(rj) > 0.0f;
           }
         }
       }
@@ -1650,11 +1667,12 @@ __device__ __forceinline__ void wave_pairs(const Agents<T> &A, const Work &W, co
       if (lane < m) {
         const int j = S.cand[cnt + lane], o = S.own[cnt + lane];
         if constexpr (MODEL == 0) {
-          const double2 xj = N.pos[j], xi = S.pos[o];
-          const V2<T> vj = N.vel[j], vi = S.vel[o];
+          const NbrState<T> nb = N.circular(j);
+          const double2 xi = S.pos[o];
+          const V2<T> vi = S.vel[o];
           T px, py;
-          if (pair_circular<T>((T)(xi.x - xj.x), (T)(xi.y - xj.y), vi.x - vj.x, vi.y - vj.y,
-                               (T)(S.r[o] + A.radius[j]), S.owner(o), px, py)) {
+          if (pair_circular<T>((T)(xi.x - nb.pos.x), (T)(xi.y - nb.pos.y), vi.x - nb.vel.x,
+                               vi.y - nb.vel.y, (T)(S.r[o] + nb.r), S.owner(o), px, py)) {
             S.sum.add(0, o, px);
             S.sum.add(1, o, py);
           }
@@ -1813,7 +1831,7 @@ __global__ void __launch_bounds__(256, MODEL == 0 ? 3 : 2) k_forces_direct(Agent
   }
   wave_fence();
   if (ok)
-    wave_pairs<T, MODEL>(A, W, FUSED ? nbr_snapshot<T>(W) : nbr_agents(A),
+    wave_pairs<T, MODEL>(A, W, FUSED ? nbr_snapshot<T>(A, W) : nbr_agents(A),
                          W.count + (size_t)p * W.cap, d, nx, ny, origin, slack, slow, L, have, i, c,
                          pos, vel, ri, S);
   if (FUSED && (fa.flags & CD_USE_OBSTACLE)) {  // wall contacts join the same exact sums
@@ -1929,10 +1947,15 @@ __device__ bool tile_region(const Agents<T> &A, const Work &W, const FusedArgs &
   // 3. neighbour data
   for (int e = tid; e < M; e += kTileThreads) {
     const int j = S.id[e];
-    S.pos[e] = cx.N.pos[j];
-    S.vel[e] = cx.N.vel[j];
-    S.r[e] = A.radius[j];
-    if constexpr (MODEL == 1) {
+    if constexpr (MODEL == 0) {
+      const NbrState<T> o = cx.N.circular(j);
+      S.pos[e] = o.pos;
+      S.vel[e] = o.vel;
+      S.r[e] = o.r;
+    } else {
+      S.pos[e] = cx.N.pos[j];
+      S.vel[e] = cx.N.vel[j];
+      S.r[e] = A.radius[j];
       S.ls[e] = cx.N.ls[j];
       S.rs[e] = cx.N.rs[j];
       S.rt[e] = A.r_t[j];
@@ -2039,7 +2062,7 @@ __global__ void __launch_bounds__(kTileThreads) k_forces_tiled(Agents<T> A, Work
   if (!FUSED && !ok) return;
   TileCtx<T> cx;
   cx.count = W.count + (size_t)p * W.cap;
-  cx.N = FUSED ? nbr_snapshot<T>(W) : nbr_agents(A);
+  cx.N = FUSED ? nbr_snapshot<T>(A, W) : nbr_agents(A);
   cx.dt = FUSED ? ss->dt : 0.0;
   cx.reset = reset;
   stage_walls(fa, d, sseg, FUSED);
