@@ -443,10 +443,14 @@ int cd_distance_map(const double *phi, const uint8_t *mask, int64_t rows, int64_
   // Passes are sent in batches, with one look at the marks after each: a
   // look waits for the stream (about 40 us), a pass without marks takes 3 us.
   // An open domain takes about as many passes as the front crosses tiles,
-  // half of tiles.x + tiles.y; what obstacles add comes in batches of eight.
+  // half of tiles.x + tiles.y; what obstacles add comes in batches of eight, or
+  // of fewer where there are few tiles: a lone tile is settled by its first
+  // pass (12 x 7 nodes: 72 us with a look after each pass, 88 in eights, 37
+  // so).
   int h_live = 1;
-  int64_t batch = std::max<int64_t>(8, ((int64_t)tiles.x + tiles.y) / 2);
-  for (int64_t pass = 0; pass < max_passes && h_live; batch = 8) {
+  const int64_t least = std::min<int64_t>(8, 2 * (int64_t)M.tiles - 1);
+  int64_t batch = std::max(least, ((int64_t)tiles.x + tiles.y) / 2);
+  for (int64_t pass = 0; pass < max_passes && h_live; batch = least) {
     const int64_t end = std::min(max_passes, pass + batch);
     for (; pass < end; ++pass)
       hipLaunchKernelGGL(relax, tiles, dim3(kFThreads), 0, s, (int)rows, (int)cols, dx, out,
