@@ -942,13 +942,14 @@ __global__ void __launch_bounds__(256) k_step_begin(Agents<T> A, Work W, Batch B
   const bool bin = binning && g.ok;
   // steps that rebuild the force kernel's processing order keep the slot ranks
   const bool ranks = W.order_every > 0 && step % (uint64_t)W.order_every == 0ull;
+  V2<T> *snap_vel = (V2<T> *)W.snap_vel;
   // an agent's snapshot and slot atomic (bin_begin), then its slot list
   // entry and neighbour record (bin_end)
   auto bin_begin = [&](int i, double2 pos, V2<T> vel, int &c, int &k, double &ri) {
     constexpr bool kPacked = MODEL == 0 && sizeof(T) == 4;
     if (!kPacked) {
       W.snap_pos[i] = pos;
-      ((V2<T> *)W.snap_vel)[i] = vel;
+      snap_vel[i] = vel;
     }
     if (MODEL) {
       const double2 ls = A.ls[i], rs = A.rs[i];
@@ -958,8 +959,8 @@ __global__ void __launch_bounds__(256) k_step_begin(Agents<T> A, Work W, Batch B
       W.snap_off[i] = shoulder_offset(A.r_ts[i], A.phi[i]);
     } else {
       ri = bin ? A.radius[i] : 0.0;
+      if (kPacked) ((NbrState<T> *)W.snap_pos)[i] = NbrState<T>{pos, vel, ri};
     }
-    if (kPacked) ((NbrState<T> *)W.snap_pos)[i] = NbrState<T>{pos, vel, ri};
     c = -1;
     k = 0;
     if (bin) {
