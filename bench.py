@@ -72,28 +72,29 @@ def pair_tally(arr, cell, segments):
 
 def step_begin_bytes(n, cells, real_bytes=8):
     """First kernel of the step, per agent.  Binning: read the position 16,
-    write the cell index, the slot and the id in the slot list (4 + 4 + 4),
-    read-modify-write the cell's count 8.  Own terms: read mass,
-    fluctuation sigma, tau_adj, target speed and target 40, the four
-    potential values of the bilinear navigation lookup 32, force, velocity
-    and target direction (2 reals each); write force and target direction
-    (2 reals each).  For the force kernel: write the snapshot (position 16,
-    velocity 2 reals) and the slot's neighbour record (24, radius read 8).
-    156 + 12 reals = 252 B/agent in fp64, 204 B in fp32; plus clearing the
-    previous step's cell counts, 4 B per grid cell."""
-    return n * (36 + 40 + 32 + 16 + 32 + 12 * real_bytes) + 4 * cells
+    write the cell index and the id in the slot list (4 + 4), read-modify-
+    write the cell's count 8.  Own terms: read mass, fluctuation sigma,
+    tau_adj, target speed and target 40, the four potential values of the
+    bilinear navigation lookup 32, force, velocity and target direction (2
+    reals each); write force and target direction (2 reals each).  For the
+    force kernel, which moves agents while others read them: read the radius
+    8, write what a neighbour is read for, once (position 16, velocity 2
+    reals, radius 8; the gate's records repeat it and count as measured
+    traffic only).  136 + 12 reals = 232 B/agent in fp64, 184 B in fp32; plus
+    clearing the previous step's cell counts, 4 B per grid cell."""
+    return n * (32 + 40 + 32 + 32 + 12 * real_bytes) + 4 * cells
 
 
 def forces_bytes(n, real_bytes=8):
     """Force kernel with the integrator (circular, fused), per agent: read
-    position 16, cell index and own slot 4 + 4, radius, mass and the five
-    pair and contact parameters 56, target speed 8, velocity, force and
-    previous force (2 reals each), and once as a neighbour its record 24
-    and its position 16, velocity 2 reals and radius 8; write position 16,
-    velocity, previous force and the reset force (2 reals each).  152 + 14 reals =
-    264 B/agent in fp64, 208 B in fp32 (neighbour data counted once: every
-    agent is read as a neighbour from cache)."""
-    return n * (16 + 8 + 56 + 8 + 24 + 16 + 8 + 16 + 14 * real_bytes)
+    position 16, cell index 4, radius, mass and the five pair and contact
+    parameters 56, target speed 8, velocity, force and previous force (2 reals
+    each), and once as a neighbour its position 16, velocity 2 reals and
+    radius 8; write position 16, velocity, previous force and the reset force
+    (2 reals each).  124 + 14 reals = 236 B/agent in fp64, 180 B in fp32
+    (neighbour data counted once, whatever the kernel reads it from or how
+    often)."""
+    return n * (16 + 4 + 56 + 8 + 16 + 8 + 16 + 14 * real_bytes)
 
 
 def measured_traffic(kernel, threads):
