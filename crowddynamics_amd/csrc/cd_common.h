@@ -111,7 +111,11 @@ inline int64_t max_blocks_e(int64_t n, int64_t S) { return n / kMinForceAgents +
 // take 40.5 us at 4 lanes, 33.9 at 8 and 39.3 at 16; at 0.6 m (3 candidates)
 // 25.9, 28.0 and 33.9.  Over that, long stencils stay with 4 lanes and short
 // ones with 2: 100000 agents at 3.6 m 123 us at 2, 98 at 4 and 99 at 8;
-// 200000 agents at 0.6 m 70 at 2 and 77 at 4.
+// 200000 agents at 0.6 m 70 at 2 and 77 at 4.  (Circular agents, fp64, spread
+// evenly.  The mean does not see a crowd packed into part of its grid, whose
+// stencils are longer: 200000 agents at 3 / m^2 in a ninth of it, 0.6 m, take
+// 86 and 86 us at 2 and 4 lanes in fp64, 74 and 70 in fp32, and with three
+// circles 159 and 166, 134 and 138.)
 inline int agent_lanes(const cd_workspace_t *w) {
   if (w->agent_lanes > 0) return (int)w->agent_lanes;
   constexpr int64_t kOnePerSimd = 64 * 1024, kOneRound = 3 * kOnePerSimd;

@@ -69,9 +69,13 @@ __device__ __forceinline__ double max_num(double a, double b) {
   return r;
 }
 
-// The correctly rounded square root of x in [2^-760, 2^1000]: the hardware
-// reciprocal root and Goldschmidt steps, without the scaling that sqrt adds
-// for the rest of the range.
+// The square root of x in [2^-760, 2^1000]: the hardware's reciprocal root
+// refined by Goldschmidt's iteration and two residual corrections, the steps
+// of LLVM's published lowering of the fp64 square root for these targets, here
+// without the scaling that it adds for the rest of the range.  Equal to sqrt,
+// bit for bit, on 1.7e10 inputs on the device: random ones over the range and
+// over one octave, and the neighbours of squares and of the squares of
+// midpoints between two doubles.
 __device__ __forceinline__ double sqrt_mid(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y, h = 0.5 * y;
@@ -154,26 +158,27 @@ __global__ void __launch_bounds__(256) k_field_init(const double *phi, const uin
 // border (or the tile itself, when the rounds ran out).
 //
 // Bound by the front's serial chain: a sweep moves it two nodes, and half a
-// sweep is one LDS round trip and one square root (605 cycles; with both
-// branches of the update selected instead of taken, minima without
-// canonicalising and a square root without scaling, and the tile read
-// together with its mark, the maps below take 1.36 ms instead of 1.65, those
-// of a 311 x 156 grid 0.67 instead of 0.80).  A visit takes some 11 rounds.
-// Against 1.30 ms on another card, shorter visits (5 rounds: 1.50), tiles of
-// 64 x 32 or 16 x 16 nodes (1.71, 1.66), the colours in arrays of their own
-// (1.35) and skipping waves with nothing new nearby (1.52) were slower.
-// Each thread owns one node of each colour (with four nodes per thread, half
-// of them of the wrong colour, the lanes idled through the other half); a
-// node whose neighbours' minima are those of its last update skips the
-// update; and the waves meet at a barrier only every fourth sweep.  Between barriers a wave
-// reads its neighbours' rows as they are at that moment: values only
-// decrease and are stored whole, so an old value is one that a later sweep
-// replaces, and a round in which no thread of the block changed a node
-// checked every node against final values.  One, two, four and eight sweeps
-// per barrier took 1.59, 1.59, 1.54 and 1.61 ms for the two maps, fill and
-// blending of a 1001 x 501 grid with 24 obstacles (host work included); all
-// tiles visited in every pass, four barriers a sweep and a wait for the
-// host after each pass took 5.8 to 6.0 ms.
+// sweep is one LDS round trip and one square root.  Each thread owns one node
+// of each colour (with four nodes per thread, half of them of the wrong colour,
+// the lanes idled through the other half); a node whose neighbours' minima are
+// those of its last update skips the update; and the waves meet at a barrier
+// only every fourth sweep.  Between barriers a wave reads its neighbours' rows
+// as they are at that moment: values only decrease and are stored whole, so an
+// old value is one that a later sweep replaces, and a round in which no thread
+// of the block changed a node checked every node against final values.
+//
+// Two maps, fill and blending of a 1001 x 501 grid with 24 obstacles, host
+// work included, each step against the one before it on one card: all tiles
+// visited in every pass, four barriers a sweep and a look after each pass 5.9
+// ms, marked tiles in batches 1.55 (one, two, four and eight sweeps a barrier
+// 1.59, 1.59, 1.54 and 1.61); both branches of the update selected instead of
+// taken, minima without canonicalising, a square root without scaling and the
+// tile read together with its mark 1.65 to 1.36.  From there shorter visits of
+// 5 rounds took 15 % more, tiles of 64 x 32 nodes 32 %, of 16 x 16 28 %, the
+// colours in arrays of their own 4 %, skipping waves with nothing new nearby
+// 17 %.  Reading a tile before its mark is known streams the map through every
+// pass, also for tiles that leave at once: 4001 x 2001 nodes take 4.7 ms a map
+// (15.5 with every tile swept in every pass).
 template <bool MID>
 __global__ void __launch_bounds__(kFThreads) k_field_relax(int rows, int cols, double dx,
                                                            double *u, const uint8_t *state,

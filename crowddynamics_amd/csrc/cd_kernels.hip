@@ -400,8 +400,7 @@ __device__ __forceinline__ void walls_each(const WallSelf<T> &me, int model, dou
 // AgentObstacleInteractions node: walls in the reference's order.
 //
 // Bound by the distance of the three circles to a segment (divisions and
-// square roots, some 1500 instructions), which a wave evaluates wherever one
-// of its lanes needs it.  kWallLanes lanes serve an agent and first test a
+// square roots), which a wave evaluates wherever one of its lanes needs it.  kWallLanes lanes serve an agent and first test a
 // segment's box against the agent's reach (walls_each), so a wave evaluates
 // about one segment in all; the few contacts are then added one after the
 // other in segment order.  One thread per agent evaluating each segment took
@@ -475,17 +474,19 @@ __global__ void __launch_bounds__(256) k_walls(Agents<T> A, int model, const dou
 // K_e: forces (owner-computes over the 3x3 cell stencil)
 // ---------------------------------------------------------------------------
 //
-// L = 2, 4, 8, 16, 32 or 64 lanes serve one agent: the candidates of its 3 x 3 cell
-// stencil, taken as one sequence, are split evenly over the lanes, and so
-// are the wall segments.  (The agent's own terms were added by the step's
-// first kernel.)  Pair and wall terms are
-// summed exactly (Fix128), so the result does not depend on the order in
-// which the binning inserted agents into cells or on how lanes and
+// L = 2, 4, 8, 16, 32 or 64 lanes serve one agent; they share the candidates
+// of its 3 x 3 cell stencil, taken as one sequence, and the wall segments.
+// (The agent's own terms were added by the step's first kernel.)  Pair and
+// wall terms are summed exactly (Fix128), so the result does not depend on the
+// order in which the binning inserted agents into cells or on how lanes and
 // workgroups split the work; it is the correctly rounded sum of the terms up
 // to the 2^-64 N grid.  Two kernels share this per-agent work:
 //
-//  * direct: workgroups take 16..64 agents in agent order; neighbour ids
-//    come from the cells' slot lists and neighbour data is read by id.
+//  * direct: workgroups take the agents in agent order, or in cell order
+//    (order_every).  The lanes deal themselves the candidates' records
+//    (NbrRec, which hold the ids) and test them with a gate; pairs that pass
+//    are evaluated from a queue of the wave, neighbour data read by id
+//    (wave_pairs).
 //  * tiled: a workgroup takes a tile of tile_x * tile_y grid cells and
 //    stages the tile plus a one-cell halo in LDS (cell counts -> offsets by
 //    a block scan -> ids from the slot lists -> neighbour data by id), then
@@ -503,7 +504,11 @@ constexpr int kTileThreads = 256;
 constexpr int kTileGroups = kTileThreads / 4;  // agents served at once
 constexpr int kTileMaxDim = 16;
 constexpr int kRegionMax = (kTileMaxDim + 2) * (kTileMaxDim + 2);
-constexpr int kWallTile = 128;  // wall segments staged in LDS at once (4 KB)
+// Wall segments staged in LDS at once (4 KB).  More are staged in turn: 64
+// rooms of 4000 agents at most, fp32, take 54 us a step with 24 segments each,
+// 71 with 184, 79 with 256 and 101 with 604 (89, 95, 99 and 123 with 256 staged
+// at once beside their frames and boxes, before the pair queue).
+constexpr int kWallTile = 128;
 
 // LDS capacity (agents of a region): nine cells of up to 128 (circular) or
 // 56 (three-circle) agents fit, so a 3 x 3 region fits whenever no cell
@@ -1514,19 +1519,22 @@ struct WaveLds {
 //
 // The lanes of an agent walk its 3 x 3 stencil, consecutive candidates on
 // consecutive lanes, and test each one with the gate (pair_gate): it needs
-// only products and passes every pair that can add a term.  Those that pass join the wave's
-// queue, and whenever 64 wait there (and at the end) every lane evaluates
-// one of them, for whichever agent it belongs to.  The sums are exact, so
-// neither who evaluates a pair nor when changes a result.
+// only products and passes every pair that can add a term.  Those that pass
+// join the wave's queue, and whenever 64 wait there (and at the end) every
+// lane evaluates one of them, for whichever agent it belongs to.  The sums are
+// exact, so neither who evaluates a pair nor when changes a result.
 //
-// Bound by the instructions of the walk and the gate, some 45 a candidate,
-// of which the search for its cell is a third (256 rooms at 4 lanes: the vector
-// units 89 % busy).  A pair in sight adds a term only if the two are on a
+// Bound by the instructions of the walk and the gate (256 rooms at 4 lanes:
+// the vector units issue 91 % of the time, 67 instructions a candidate for the
+// whole kernel, 16 of them the search for its cell).  A pair in sight adds a term only if the two are on a
 // collision course or touch: 3 % of the candidates at cells of sight + 2 r,
 // a fifth at 0.6 m.  Evaluating pairs where they were met, a wave ran the pair
-// function (300 instructions in fp64) for nearly every candidate of its
-// busiest lane.  256 rooms, fp32: 449 us with fp64 records and a branch
-// for each lane's end, 280 now.  Walking the three rows of cells one after
+// function for nearly every candidate of its busiest lane.  256 rooms, fp32:
+// 449 us with fp64 records and a branch for each lane's end, 273 now.  Where
+// nearly every candidate passes, the second read costs more than the gate
+// saves: a million agents at 3 / m^2 in cells of 0.6 m take 359 us a step in
+// fp32, and 322 with each pair evaluated from a record of its own data (at
+// 2 / m^2 292 and 291).  Walking the three rows of cells one after
 // the other (two comparisons a candidate instead of eight) idles lanes at
 // each row's end and was slower (1835 against 1690 us for five steps), and so
 // was fetching one half of a round while the other is gated (2008).
