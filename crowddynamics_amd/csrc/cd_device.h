@@ -548,11 +548,15 @@ __device__ __forceinline__ double2 shoulder_offset(double r_ts, double phi) {
 
 // A radius about the torso's centre that holds the three circles of an
 // agent (the hardware square root is within 2^-24; the margin covers it).
+// Infinite where a shoulder is not finite: a pair in sight then has a NaN
+// torque from a moment arm times no force.
 __device__ __forceinline__ double tc_reach(double2 p, double2 ls, double2 rs, double r_t,
                                            double r_s) {
   const double lx = ls.x - p.x, ly = ls.y - p.y, rx = rs.x - p.x, ry = rs.y - p.y;
-  const double o2 = fmax(lx * lx + ly * ly, rx * rx + ry * ry);
-  return fmax(fabs(r_t), __builtin_amdgcn_sqrt(o2) * (1.0 + 0x1p-20) + fabs(r_s));
+  const double l2 = lx * lx + ly * ly, r2 = rx * rx + ry * ry;
+  const double body =
+      fmax(fabs(r_t), __builtin_amdgcn_sqrt(fmax(l2, r2)) * (1.0 + 0x1p-20) + fabs(r_s));
+  return l2 + r2 < __builtin_inf() ? body : __builtin_inf();
 }
 
 // interaction_agent_agent_three_circle (core/interactions.py:73-104) in the

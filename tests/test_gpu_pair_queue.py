@@ -6,8 +6,11 @@ fill several times and ones that stay empty, and shoulders anywhere."""
 import numpy as np
 import pytest
 
+from crowddynamics_amd import core
 from crowddynamics_amd.agents import empty_agents
+from crowddynamics_amd.device import DeviceAgents, Workspace
 from crowddynamics_amd.stepper import Stepper
+from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -65,3 +68,35 @@ def test_queue_equals_every_candidate(model, precision, n, side, cell, slots):
         if model == 'three_circle':
             for f in ('orientation', 'angular_velocity', 'torque_prev'):
                 assert np.array_equal(got[f], want[f]), (lanes, f)
+
+
+@pytest.mark.filterwarnings('ignore')
+@pytest.mark.parametrize('value', [np.nan, np.inf, 1e200])
+def test_shoulders_that_are_not_finite(value):
+    """A shoulder that is not finite gives its pairs in sight a NaN torque,
+    also where their force is zero: the agents the oracle names, and the same
+    from the queue as from every candidate."""
+    n = 80
+    arr = _agents('three_circle', n, 6.0, 5)
+    off = 0.15 * np.stack([np.sin(arr['orientation']), -np.cos(arr['orientation'])], 1)
+    arr['position_ls'], arr['position_rs'] = arr['position'] - off, arr['position'] + off
+    arr['position_ls'][::13, 0] = value
+    arr['position_rs'][5, 1] = value
+    want = arr.copy()
+    with np.errstate(all='ignore'):
+        O.agent_agent_block_list(want, 3.6)
+    for f in ('force', 'torque'):  # the exact sums hold terms below 2^62, a larger one is NaN
+        want[f][~(np.abs(want[f]) < 2.0 ** 62)] = np.nan
+    assert 0 < np.sum(np.isnan(want['torque'])) < n
+    dev = DeviceAgents(arr.copy())
+    core.agent_agent_block_list(dev, 3.6, Workspace(n, 64, 1, cell_slots=64))
+    got = arr.copy()
+    dev.download(got)
+    assert np.array_equal(np.isnan(got['torque']), np.isnan(want['torque']))
+    assert np.array_equal(np.isnan(got['force']), np.isnan(want['force']))
+    kw = dict(cell_size=3.6, bounds=(-4.0, -4.0, 10.0, 10.0))
+    every = _run(arr, 1, tile=(2, 2), **kw)
+    for lanes in (2, 16):
+        out = _run(arr, 1, lanes=lanes, **kw)
+        for f in ('force_prev', 'torque_prev', 'orientation'):
+            assert np.array_equal(out[f], every[f], equal_nan=True), (lanes, f)
